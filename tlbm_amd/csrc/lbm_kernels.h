@@ -35,6 +35,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <utility>
+
 #include "lattice.h"
 #include "mlp.h"
 #include "udiv.h"
@@ -64,6 +66,14 @@ template <int ST> constexpr bool kClosureNTLoad = (ST == ST_F16);
 // (6).  FP32 D3Q27 stays at 4: at 5 it spills (325 against 299 us).
 template <int ST, int Q>
 constexpr int kClosureWaves = Q == 27 ? (ST == ST_F16 ? 5 : 4) : (ST == ST_F32 && Q == 19 ? 5 : 6);
+// Waves per SIMD the step is register-allocated for (least and most).  FP16
+// left alone takes 96 VGPRs for D3Q19 (114 against 102 us per step); FP32
+// D3Q19, HBM-bound, loses with more than 5 (68 VGPRs, 7 waves: 206.7 against
+// 202.6 us).
+template <int ST, int Q>
+constexpr int kStepWaves = ST == ST_F16 ? (Q == 27 ? 6 : 8) : ST == ST_F32 && Q == 15 ? 8 : 1;
+template <int ST, int Q>
+constexpr int kStepWavesMax = ST == ST_F32 && Q == 19 ? 5 : 8;
 // Steps with kTypeAhead, and the closure collide in every storage, load the
 // chunk's common node type (or the node's own) ahead of their gathers, so
 // that it lands with them; loaded after them it costs each wavefront one
@@ -112,6 +122,9 @@ struct StepArgs {
     int dynamics;      // 1: BGK relaxation, other values: none (TLBM_Partition.cpp:795-807)
     int smag;          // cs > 0
     double cs, omega, nu, nu2, u_bc, rho_bc, inv_1mu, inv_rho_bc;
+    struct {           // the same as float, for the FP32 arithmetic
+        float cs, omega, nu, nu2, u_bc, rho_bc, inv_1mu, inv_rho_bc;
+    } fl;
     double w[27];      // weights (the reference's float-literal values unless exact)
     float wf[27];      // the same weights as float (FP32/FP16 compute)
     float h_scale[27];     // FP16 storage: h = d * h_scale (= d / w)
@@ -145,6 +158,23 @@ struct StepArgs {
     // per-node inlet velocity u_z(x, y) (nx*ny values), or null for u_bc
     const float *inlet_uz;
 };
+
+// A scalar argument in the compute type: converting the double on the GPU
+// would cost a vector register each (there is no scalar conversion).
+template <class T>
+__device__ inline T num(double d, float f) {
+    if constexpr (sizeof(T) == 8) return d; else return f;
+}
+
+// The first direction with the weight of s.  Weights are read by it, so that
+// a kernel holds one register per distinct weight, not one per direction.
+template <class L>
+constexpr int weight_class(int s) {
+    auto order = [](int k) { return L::ex[k] * L::ex[k] + L::ey[k] * L::ey[k] + L::ez[k] * L::ez[k]; };
+    int k = 0;
+    while (order(k) != order(s)) ++k;
+    return k;
+}
 
 // Offset of population s of node g in a state buffer (chunked layout).
 template <int Q>
@@ -492,6 +522,27 @@ struct PushOut {
     }
 };
 
+// f(integral_constant k) for k = A .. B - 1: an unrolled loop whose index is a
+// constant in the body.  Register arrays are indexed by it: a loop variable
+// becomes a constant only after unrolling, and an array that the compiler has
+// not split into scalars by then is kept as one tuple of registers, which
+// every branch copies whole.
+template <int A, class F, int... I>
+__device__ inline void each_impl(F &&f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, A + I>{}), ...);
+}
+template <int A, int B, class F>
+__device__ inline void each(F &&f) {
+    each_impl<A>(f, std::make_integer_sequence<int, B - A>{});
+}
+// ... for the first direction of every pair of opposite directions.
+template <class L, class F>
+__device__ inline void each_pair(F &&f) {
+    each<1, L::Q>([&](auto k) {
+        if constexpr (k < L::bb[k]) f(k);
+    });
+}
+
 // a * b + c rounded once.
 __device__ inline float fma_t(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ inline double fma_t(double a, double b, double c) { return __builtin_fma(a, b, c); }
@@ -529,8 +580,7 @@ __device__ inline bool node_prepare(T (&f)[L::Q], T (&feq)[L::Q], int t, T &rho,
     // compute_macroscopic_data, LatticeStructure.hpp:69-90
     {
         T r = T(-0.0), mx = T(-0.0), my = T(-0.0), mz = T(-0.0);
-#pragma unroll
-        for (int s = 0; s < Q; ++s) {
+        each<0, Q>([&](auto s) {
             if constexpr (SC) {
                 r = fma_t(w[s], f[s], r);
                 if (L::ex[s] > 0) mx = fma_t(w[s], f[s], mx); else if (L::ex[s] < 0) mx = fma_t(-w[s], f[s], mx);
@@ -542,7 +592,7 @@ __device__ inline bool node_prepare(T (&f)[L::Q], T (&feq)[L::Q], int t, T &rho,
                 if (L::ey[s] > 0) my += f[s]; else if (L::ey[s] < 0) my -= f[s];
                 if (L::ez[s] > 0) mz += f[s]; else if (L::ez[s] < 0) mz -= f[s];
             }
-        }
+        });
         if constexpr (SHIFT) {
             dlt = r + (sizeof(T) == 8 ? T(a.dw_d) : T(a.dw));
             rho = T(1) + dlt;
@@ -565,36 +615,36 @@ __device__ inline bool node_prepare(T (&f)[L::Q], T (&feq)[L::Q], int t, T &rho,
         ux = T(0); uy = T(0); uz = T(0);
         if (COLLIDE) {
             T g[Q];
-#pragma unroll
-            for (int s = 0; s < Q; ++s) g[s] = f[L::bb[s]];
-#pragma unroll
-            for (int s = 0; s < Q; ++s) {
+            each<0, Q>([&](auto s) {
+                g[s] = f[L::bb[s]];
+            });
+            each<0, Q>([&](auto s) {
                 f[s] = g[s];
                 feq[s] = g[s];
-            }
+            });
         }
         return false;
     }
     if (t == 2) {
         // set_inletW_bc_macro (D3Q19LatticeStructure.hpp:108-132)
         T s_in = T(-0.0), sz = T(-0.0);
-#pragma unroll
-        for (int i = 0; i < L::n_unk; ++i)
+        each<0, L::n_unk>([&](auto i) {
             s_in = SC ? fma_t(w[L::in_list[i]], f[L::in_list[i]], s_in) : s_in + f[L::in_list[i]];
-#pragma unroll
-        for (int i = 0; i < L::n_zero; ++i)
+        });
+        each<0, L::n_zero>([&](auto i) {
             sz = SC ? fma_t(w[L::zero_list[i]], f[L::zero_list[i]], sz) : sz + f[L::zero_list[i]];
+        });
         ux = T(0); uy = T(0);
         const T c_in0 = sizeof(T) == 8 ? T(a.c_in_d) : T(a.c_in);
-        T inv_1mu = T(a.inv_1mu), c_in = c_in0;
+        T inv_1mu = num<T>(a.inv_1mu, a.fl.inv_1mu), c_in = c_in0;
         if (a.inlet_uz) {
             // a prescribed inlet profile: 1/(1-u) and the deviation constant per node
             const T u = T(a.inlet_uz[g % a.nxny]);
             uz = u;
             inv_1mu = T(1) / (T(1) - u);
-            c_in = c_in0 + (u - T(a.u_bc));
+            c_in = c_in0 + (u - num<T>(a.u_bc, a.fl.u_bc));
         } else {
-            uz = T(a.u_bc);
+            uz = num<T>(a.u_bc, a.fl.u_bc);
         }
         if constexpr (SHIFT) {
             dlt = inv_1mu * (c_in + (T(2) * s_in + sz));
@@ -605,33 +655,32 @@ __device__ inline bool node_prepare(T (&f)[L::Q], T (&feq)[L::Q], int t, T &rho,
     } else if (t == 3) {
         // set_outletE_bc_macro (D3Q19LatticeStructure.hpp:135-156); ux, uy kept
         T s_out = T(-0.0), sz = T(-0.0);
-#pragma unroll
-        for (int i = 0; i < L::n_unk; ++i)
+        each<0, L::n_unk>([&](auto i) {
             s_out = SC ? fma_t(w[L::out_list[i]], f[L::out_list[i]], s_out) : s_out + f[L::out_list[i]];
-#pragma unroll
-        for (int i = 0; i < L::n_zero; ++i)
+        });
+        each<0, L::n_zero>([&](auto i) {
             sz = SC ? fma_t(w[L::zero_list[i]], f[L::zero_list[i]], sz) : sz + f[L::zero_list[i]];
-        rho = T(a.rho_bc);
+        });
+        rho = num<T>(a.rho_bc, a.fl.rho_bc);
         if constexpr (SHIFT) {
             dlt = sizeof(T) == 8 ? T(a.rho_bc - 1.0) : T(a.drho_bc);
-            uz = T(a.inv_rho_bc) * ((sizeof(T) == 8 ? T(a.c_out_d) : T(a.c_out)) + (T(2) * s_out + sz));
+            uz = num<T>(a.inv_rho_bc, a.fl.inv_rho_bc) * ((sizeof(T) == 8 ? T(a.c_out_d) : T(a.c_out)) + (T(2) * s_out + sz));
         } else {
-            uz = T(-1) + T(a.inv_rho_bc) * (T(2) * s_out + sz);
+            uz = T(-1) + num<T>(a.inv_rho_bc, a.fl.inv_rho_bc) * (T(2) * s_out + sz);
         }
     }
     if (!COLLIDE) return true;
     if (t == 5) {
         // set_uz_bc (LatticeStructure.hpp:166-177); the y term reads uy of
         // node s of this step, as the reference's uy[spd] does
-        const T ubc = a.inlet_uz ? T(a.inlet_uz[g % a.nxny]) : T(a.u_bc);
-#pragma unroll
-        for (int s = 1; s < Q; ++s) {
+        const T ubc = a.inlet_uz ? T(a.inlet_uz[g % a.nxny]) : num<T>(a.u_bc, a.fl.u_bc);
+        each<1, Q>([&](auto s) {
             T br = T(-0.0);
             if (L::ez[s] > 0) br += (ubc - uz); else if (L::ez[s] < 0) br -= (ubc - uz);
             if (L::ex[s] > 0) br -= ux; else if (L::ex[s] < 0) br += ux;
             if (L::ey[s] > 0) br -= uy_head[s]; else if (L::ey[s] < 0) br += uy_head[s];
             f[s] = SC ? f[s] + T(3) * rho * br : f[s] + T(3) * rho * w[s] * br;
-        }
+        });
     }
     // compute_equilibrium, LatticeStructure.hpp:92-103
     {
@@ -664,29 +713,27 @@ __device__ inline bool node_prepare(T (&f)[L::Q], T (&feq)[L::Q], int t, T &rho,
                 Uy = t3 * rho * uy;
                 Uz = t3 * rho * uz;
             }
-#pragma unroll
-            for (int s = 0; s < Q; ++s) {
+            each<0, Q>([&](auto s) {
                 const T t = (s == 0) ? T(0) : edot<T>(L::ex[s], L::ey[s], L::ez[s], Ux, Uy, Uz);
                 feq[s] = SC ? A + t * (T(1) + t * h) : w[s] * (A + t * (T(1) + t * h));
-            }
+            });
             const T corr = rho * (T(1.5) * T(a.dk1) * usq - T(a.dk0));
             feq[0] += SC ? corr * T(a.h_scale[0]) : corr;
         } else {
-#pragma unroll
-            for (int s = 0; s < Q; ++s) {
+            each<0, Q>([&](auto s) {
                 const T cu = (s == 0) ? T(0) : T(3) * edot<T>(L::ex[s], L::ey[s], L::ez[s], ux, uy, uz);
                 feq[s] = w[s] * rho * (T(1) + cu + T(0.5) * (cu * cu) - T(1.5) * usq);
-            }
+            });
         }
     }
     if (t == 2) {
-#pragma unroll
-        for (int i = 0; i < L::n_unk; ++i)
+        each<0, L::n_unk>([&](auto i) {
             f[L::in_unk[i]] = feq[L::in_unk[i]] + f[L::in_par[i]] - feq[L::in_par[i]];
+        });
     } else if (t == 3) {
-#pragma unroll
-        for (int i = 0; i < L::n_unk; ++i)
+        each<0, L::n_unk>([&](auto i) {
             f[L::out_unk[i]] = feq[L::out_unk[i]] + f[L::out_par[i]] - feq[L::out_par[i]];
+        });
     }
     return true;
 }
@@ -701,10 +748,9 @@ template <class L, class T, bool SC = false>
 __device__ inline void node_stress(const T (&f)[L::Q], const T (&feq)[L::Q], T (&pi)[6],
                                    const T (&w)[L::Q]) {
     T sxx = T(-0.0), syy = T(-0.0), szz = T(-0.0), sxy = T(-0.0), sxz = T(-0.0), syz = T(-0.0);
-#pragma unroll
-    for (int s = 0; s < L::Q; ++s) {
+    each<0, L::Q>([&](auto s) {
         // the rest direction adds to no sum; the others come with their partner
-        if (SC && (s == 0 || L::bb[s] < s)) continue;
+        if constexpr (SC && (s == 0 || L::bb[s] < s)) return;
         const T fn = SC ? ((f[s] - feq[s]) + (f[L::bb[s]] - feq[L::bb[s]])) * w[s] : f[s] - feq[s];
         if (L::ex[s] != 0) sxx += fn;
         if (L::ey[s] != 0) syy += fn;
@@ -712,7 +758,7 @@ __device__ inline void node_stress(const T (&f)[L::Q], const T (&feq)[L::Q], T (
         if (L::ex[s] * L::ey[s] > 0) sxy += fn; else if (L::ex[s] * L::ey[s] < 0) sxy -= fn;
         if (L::ex[s] * L::ez[s] > 0) sxz += fn; else if (L::ex[s] * L::ez[s] < 0) sxz -= fn;
         if (L::ey[s] * L::ez[s] > 0) syz += fn; else if (L::ey[s] * L::ez[s] < 0) syz -= fn;
-    }
+    });
     pi[0] = sxx; pi[1] = syy; pi[2] = szz; pi[3] = sxy; pi[4] = sxz; pi[5] = syz;
 }
 
@@ -732,68 +778,298 @@ __device__ inline T smagorinsky_omega(const T (&pi)[6], const StepArgs &a) {
         static_assert(sizeof(T) == 4, "FP32 arithmetic");
         const float n2 = pi[0] * pi[0] + pi[1] * pi[1] + pi[2] * pi[2] +
                          2.f * (pi[3] * pi[3] + pi[4] * pi[4] + pi[5] * pi[5]);
-        const float P = __builtin_amdgcn_sqrtf(__builtin_amdgcn_sqrtf(n2) * float(a.cs) + float(a.nu2)) -
-                        float(a.nu);
-        return __builtin_amdgcn_rcpf(3.f * (float(a.nu) + P * (1.f / 6.f)) + 0.5f);
+        const float P = __builtin_amdgcn_sqrtf(__builtin_amdgcn_sqrtf(n2) * a.fl.cs + a.fl.nu2) -
+                        a.fl.nu;
+        return __builtin_amdgcn_rcpf(3.f * (a.fl.nu + P * (1.f / 6.f)) + 0.5f);
     }
     T P = stress_norm<T>(pi);
-    P *= T(a.cs);
-    P = sqrt(P + T(a.nu2)) - T(a.nu);
+    P *= num<T>(a.cs, a.fl.cs);
+    P = sqrt(P + num<T>(a.nu2, a.fl.nu2)) - num<T>(a.nu, a.fl.nu);
     const T nu_e = P / T(6);
-    return T(1) / (T(3) * (T(a.nu) + nu_e) + T(0.5));
+    return T(1) / (T(3) * (num<T>(a.nu, a.fl.nu) + nu_e) + T(0.5));
 }
 
 // relax, LatticeStructure.hpp:155-163.
 template <class L, class T>
 __device__ inline void node_relax(T (&f)[L::Q], const T (&feq)[L::Q], T om) {
-#pragma unroll
-    for (int s = 0; s < L::Q; ++s) f[s] = f[s] - om * (f[s] - feq[s]);
+    each<0, L::Q>([&](auto s) {
+        f[s] = f[s] - om * (f[s] - feq[s]);
+    });
 }
 
-// relax of a fluid node in FP32 storage, conserving to the rounding of
-// f - feq.  In exact arithmetic the mass and momentum of f - feq are small
-// values set by the weights (the reference's D3Q15/D3Q19 float weights do
-// not sum to 1); rounded FP32 equilibria miss them by a few ulp of feq, the
-// same amount at every node of a steady flow, and that residue accumulates
-// step after step (D3Q19 cylinder array: velocity L2 against FP64 1.6e-5
-// after 20000 steps).  The values are those of the weights w, not of their
-// float roundings: the D3Q27 weights sum to 1 in double but to 1 + 7.5e-9
-// in float, a mass source FP64 does not have.  The residue of mass m0 and
-// momentum m is taken out of f - feq as w_s (m0 + 3 e_s.m), which carries
-// that mass and momentum.
-template <class L>
-__device__ inline void node_relax_conserving(float (&f)[L::Q], const float (&feq)[L::Q],
-                                             const float (&w)[L::Q], float om, float rho,
-                                             float ux, float uy, float uz, const StepArgs &a) {
-    constexpr int Q = L::Q;
-    float nq[Q], m0 = -0.0f, mx = -0.0f, my = -0.0f, mz = -0.0f;
-#pragma unroll
-    for (int s = 0; s < Q; ++s) {
-        nq[s] = f[s] - feq[s];
-        m0 += nq[s];
-        if (L::ex[s] > 0) mx += nq[s]; else if (L::ex[s] < 0) mx -= nq[s];
-        if (L::ey[s] > 0) my += nq[s]; else if (L::ey[s] < 0) my -= nq[s];
-        if (L::ez[s] > 0) mz += nq[s]; else if (L::ez[s] < 0) mz -= nq[s];
-    }
-    m0 -= rho * (1.5f * a.k1 * (ux * ux + uy * uy + uz * uz) - a.k0);
-    const float rk = rho * a.k2;
-    mx = 3.0f * (mx - rk * ux);
-    my = 3.0f * (my - rk * uy);
-    mz = 3.0f * (mz - rk * uz);
-#pragma unroll
-    for (int s = 0; s < Q; ++s) {
-        const float c = (s == 0) ? m0 : m0 + edot<float>(L::ex[s], L::ey[s], L::ez[s], mx, my, mz);
-        f[s] = f[s] - om * (nq[s] - w[s] * c);
-    }
-}
-
-// Whether a step kernel relaxes fluid nodes with node_relax_conserving:
+// Whether a step kernel's fluid nodes relax conserving (fluid_pairs):
 // FP32 storage.  FP16's own rounding is stochastic, no bias; its float
 // weights get the mass and momentum balance of w from the equilibrium
 // corrections dt3, dk0, dk1 instead, at a fraction of the cost (the
 // conserving relax took 13 % of the FP16 D3Q27 step).
 template <int ST, int Q>
 constexpr bool kConserve = ST == ST_F32;
+
+// 1/x to within rounding: in float the hardware reciprocal (1 ulp) and one
+// Newton step (3 operations; the correctly rounded division takes 10).
+__device__ inline double rcp_newton(double x) { return 1.0 / x; }
+__device__ inline float rcp_newton(float x) {
+    const float r = __builtin_amdgcn_rcpf(x);
+    return fma_t(r, fma_t(-x, r, 1.0f), r);
+}
+
+#define TLBM_ROUND_EACH _Pragma("clang fp contract(off)")
+
+// ---- deviation storage: the node update by direction pairs ---------------------------------
+// A direction s and its opposite b = bb[s] have the same weight w and the
+// equilibria w (c + t) and w (c - t), c = A + t^2 h, so what a pair needs
+// comes from its sum and its difference: a fluid node's update takes about
+// 170 operations (D3Q19) where one direction at a time took 250.  n[] holds
+// f - feq in that form: n[0], and per pair (s < b) n[s] = n_s + n_b and
+// n[b] = n_s - n_b.  Node types other than fluid patch the fluid update
+// where a wavefront holds any (branches on the whole wavefront, so that a
+// lane's values are not kept for two sides of a branch).
+// SC: f[] and n[] hold h = d / w.
+
+// The inlet's (outlet's) unknown populations, those with e_z > 0 (< 0):
+// f_unknown = feq_unknown + f_partner - feq_partner, so the unknown's f - feq
+// is its partner's.  With the opposite direction for a partner (D3Q19, D3Q27)
+// the equilibria differ by 2 w t, with the mirror image in z (D3Q15) by
+// 2 w e_z U_z (1 + 2 h (e_x U_x + e_y U_y)).  Selects, no branches: where the
+// two sides of a branch name different elements of f, the compiler indexes
+// f by a variable, and f goes to memory or is copied whole.
+template <class L, class T, bool SC>
+__device__ inline void pairs_rebuild(T (&f)[L::Q], T (&n)[L::Q], bool inlet, bool outlet, T h, T Ux, T Uy, T Uz,
+                                     const T (&w)[L::Q]) {
+    constexpr bool kOpposite = L::in_par[1] == L::bb[L::in_unk[1]];
+    each<0, L::n_unk>([&](auto k) {
+        constexpr int s = L::in_unk[k], p = L::in_par[k];
+        const T w2 = SC ? T(2.0) : T(2.0) * w[s];
+        T d;  // feq_s - feq_p
+        if constexpr (kOpposite || L::ex[s] == 0)
+            d = w2 * edot<T>(L::ex[s], L::ey[s], L::ez[s], Ux, Uy, Uz);
+        else
+            d = w2 * Uz * fma_t(T(2.0) * h, edot<T>(L::ex[s], L::ey[s], 0, Ux, Uy, Uz), T(1.0));
+        const T fs = f[s], fp = f[p];
+        f[s] = inlet ? fp + d : fs;
+        f[p] = outlet ? fs - d : fp;
+    });
+    if constexpr (kOpposite) {
+        each<0, L::n_unk>([&](auto k) {
+            constexpr int s = L::in_unk[k], b = L::bb[s], lo = s < b ? s : b, hi = s < b ? b : s;
+            const T nb = s < b ? n[lo] - n[hi] : n[lo] + n[hi];  // 2 n_b
+            const T ns = s < b ? n[lo] + n[hi] : n[lo] - n[hi];  // 2 n_s
+            n[lo] = inlet ? nb : outlet ? ns : n[lo];
+            n[hi] = inlet || outlet ? T(0.0) : n[hi];
+        });
+    } else {
+        // D3Q15: the pairs (7, 14), (8, 13), (9, 12), (10, 11) trade members
+        // with the mirror images 7-11, 8-12, 9-13, 10-14; 5 and 6 are both
+        const T n5 = n[5] + n[6], n6 = n[5] - n[6];
+        n[5] = inlet ? n6 : outlet ? n5 : n[5];
+        n[6] = inlet || outlet ? T(0.0) : n[6];
+        each<7, 9>([&](auto k) {
+            // two pairs at a time: (s, b) and (m, q), q the mirror of s, m that of b
+            constexpr int s = k, b = L::bb[s], q = s + 4, m = L::bb[q];
+            const T xs = T(0.5) * (n[s] + n[b]), xb = T(0.5) * (n[s] - n[b]);
+            const T xm = T(0.5) * (n[m] + n[q]), xq = T(0.5) * (n[m] - n[q]);
+            const T ys = inlet ? xq : xs, ym = inlet ? xb : xm;
+            const T yb = outlet ? xm : xb, yq = outlet ? xs : xq;
+            n[s] = ys + yb;
+            n[b] = ys - yb;
+            n[m] = ym + yq;
+            n[q] = ym - yq;
+        });
+    }
+}
+
+// The step's rules up to f - feq (node_prepare's): moments, the inlet,
+// outlet and type-5 rules, equilibrium, reconstruction; fills n[].  A solid
+// node's n is finite (it takes no part in the rules).
+// CONSERVE: the rounding residue of mass and momentum in a fluid node's
+// f - feq is taken out.  In exact arithmetic f - feq has the mass and
+// momentum that the weights w set (the reference's D3Q15/D3Q19 T weights
+// do not sum to 1); rounded FP32 equilibria miss them by a few ulp of feq,
+// the same amount at every node of a steady flow, and that residue would
+// accumulate step after step (D3Q19 cylinder array: velocity L2 against FP64
+// 1.6e-5 after 20000 steps).  The targets are those of the weights w, not of
+// their T roundings: the D3Q27 weights sum to 1 in double but to
+// 1 + 7.5e-9 in float, a mass source FP64 does not have.  The residue is
+// measured on f - feq, whose own rounding is far below that of feq, and mass
+// m0 and momentum m of it are taken out as w_s (m0 + 3 e_s.m).  (The mass out
+// of the rest population and the momentum out of the axis pairs alone would
+// be 0.5 % (D3Q19) to 2 % (D3Q27) faster and as accurate, but not isotropic.)
+// The rounding of a steady FP32 flow's moments repeats every step, so every
+// operation is written out (TLBM_ROUND_EACH: products and sums are contracted
+// only where fma_t says so): both step kernels then give the same bits, and
+// the drift that tests bound is that of this source.  Of the equivalent forms
+// of the equilibrium A + t (t h +- 1) keeps a uniform flow's momentum closest
+// to FP64's (D3Q19 float weights, 4000 steps: 4e-7; A + t^2 h +- t 1 to 5e-6).
+template <class L, class T, bool SC, bool CONSERVE>
+__device__ inline void pairs_prepare(T (&f)[L::Q], T (&n)[L::Q], int t, const StepArgs &a,
+                                     const T *__restrict__ uy_head, const T (&w)[L::Q], uint32_t g) {
+    TLBM_ROUND_EACH
+    static_assert(!(SC && CONSERVE), "the conserving form works on d");
+    T r = SC ? w[0] * f[0] : f[0], mx = T(-0.0), my = T(-0.0), mz = T(-0.0);
+    each_pair<L>([&](auto k) {
+        constexpr int s = k, b = L::bb[s];
+        n[s] = f[s] + f[b];
+        n[b] = f[s] - f[b];
+        if (SC) {
+            r = fma_t(w[s], n[s], r);
+            if (L::ex[s]) mx = fma_t(T(L::ex[s]) * w[s], n[b], mx);
+            if (L::ey[s]) my = fma_t(T(L::ey[s]) * w[s], n[b], my);
+            if (L::ez[s]) mz = fma_t(T(L::ez[s]) * w[s], n[b], mz);
+        } else {
+            r += n[s];
+            if (L::ex[s] > 0) mx += n[b]; else if (L::ex[s] < 0) mx -= n[b];
+            if (L::ey[s] > 0) my += n[b]; else if (L::ey[s] < 0) my -= n[b];
+            if (L::ez[s] > 0) mz += n[b]; else if (L::ez[s] < 0) mz -= n[b];
+        }
+    });
+    T dlt = r + num<T>(a.dw_d, a.dw), rho = T(1.0) + dlt;
+    T inv = t == 1 ? T(1.0) : rcp_newton(rho);
+    const bool inlet = t == 2, outlet = t == 3, ends = __any(inlet || outlet);
+    if (ends) {
+        // set_inletW_bc_macro, set_outletE_bc_macro
+        // (D3Q19LatticeStructure.hpp:108-156); at the outlet u_x and u_y of
+        // the node's own density are kept
+        T level = T(-0.0), in = T(-0.0), out = T(-0.0);
+        each<0, L::n_zero>([&](auto k) {
+            constexpr int s = L::zero_list[k];
+            level = SC ? fma_t(w[s], f[s], level) : level + f[s];
+        });
+        each<0, L::n_unk>([&](auto k) {
+            constexpr int s = L::in_list[k], p = L::out_list[k];
+            in = SC ? fma_t(w[s], f[s], in) : in + f[s];
+            out = SC ? fma_t(w[p], f[p], out) : out + f[p];
+        });
+        const T u_bc = num<T>(a.u_bc, a.fl.u_bc), rho_bc = num<T>(a.rho_bc, a.fl.rho_bc),
+                inv_bc = num<T>(a.inv_rho_bc, a.fl.inv_rho_bc), c_out = num<T>(a.c_out_d, a.c_out);
+        T uz = u_bc, inv_1mu = num<T>(a.inv_1mu, a.fl.inv_1mu), c_in = num<T>(a.c_in_d, a.c_in);
+        if (a.inlet_uz) {
+            // a prescribed inlet profile: 1/(1-u) and the deviation constant per node
+            uz = T(a.inlet_uz[g % a.nxny]);
+            inv_1mu = T(1.0) / (T(1.0) - uz);
+            c_in += uz - u_bc;
+        }
+        const T keep = inlet ? T(0.0) : outlet ? rho_bc * inv : T(1.0);
+        dlt = inlet ? inv_1mu * (c_in + (T(2.0) * in + level)) : outlet ? num<T>(a.rho_bc - 1.0, a.drho_bc) : dlt;
+        rho = outlet ? rho_bc : T(1.0) + dlt;
+        inv = outlet ? inv_bc : inlet ? rcp_newton(rho) : inv;
+        mx *= keep;
+        my *= keep;
+        mz = inlet ? rho * uz : outlet ? rho_bc * (inv_bc * (c_out + (T(2.0) * out + level))) : mz;
+    }
+    // rho u^2 from rounded squares, as node_prepare forms it
+    const T q2 = inv * (mx * mx + my * my + mz * mz);
+    const T h = T(0.5) * inv, A = fma_t(T(-1.5), q2, dlt);
+    // FP16 (SC): 3 + dt3 times the momentum, rounded once, so that the
+    // correction (which 3 + dt3 would lose) survives rounding on average
+    const T Ux = SC ? fma_t(T(3.0), mx, T(a.dt3) * mx) : T(3.0) * mx;
+    const T Uy = SC ? fma_t(T(3.0), my, T(a.dt3) * my) : T(3.0) * my;
+    const T Uz = SC ? fma_t(T(3.0), mz, T(a.dt3) * mz) : T(3.0) * mz;
+    n[0] = SC ? f[0] - A : fma_t(-w[0], A, f[0]);
+    if (SC) n[0] -= (T(1.5) * T(a.dk1) * q2 - T(a.dk0) * rho) * T(a.h_scale[0]);
+    T m0 = n[0], cx = T(-0.0), cy = T(-0.0), cz = T(-0.0);
+    each_pair<L>([&](auto k) {
+        TLBM_ROUND_EACH
+        constexpr int s = k, b = L::bb[s];
+        const T tt = edot<T>(L::ex[s], L::ey[s], L::ez[s], Ux, Uy, Uz);
+        if (CONSERVE) {
+            // each direction's f - feq rounds once, far below f; formed from
+            // the pair's sum and difference it would carry their rounding
+            const T x = fma_t(-w[s], fma_t(tt, fma_t(tt, h, T(1.0)), A), f[s]);
+            const T y = fma_t(-w[s], fma_t(tt, fma_t(tt, h, T(-1.0)), A), f[b]);
+            n[s] = x + y;
+            n[b] = x - y;
+            m0 += n[s];
+            if (L::ex[s] > 0) cx += n[b]; else if (L::ex[s] < 0) cx -= n[b];
+            if (L::ey[s] > 0) cy += n[b]; else if (L::ey[s] < 0) cy -= n[b];
+            if (L::ez[s] > 0) cz += n[b]; else if (L::ez[s] < 0) cz -= n[b];
+        } else {
+            const T c = fma_t(tt * tt, h, A);
+            const T w2 = SC ? T(2.0) : T(2.0) * w[s];
+            n[s] = fma_t(-w2, c, n[s]);
+            n[b] = fma_t(-w2, tt, n[b]);
+        }
+    });
+    if constexpr (CONSERVE) {
+        const bool fluid = t == 0;
+        m0 = fluid ? m0 - fma_t(T(1.5) * T(a.k1), q2, -(T(a.k0) * rho)) : T(0.0);
+        cx = fluid ? T(3.0) * fma_t(-T(a.k2), mx, cx) : T(0.0);
+        cy = fluid ? T(3.0) * fma_t(-T(a.k2), my, cy) : T(0.0);
+        cz = fluid ? T(3.0) * fma_t(-T(a.k2), mz, cz) : T(0.0);
+        n[0] = fma_t(-w[0], m0, n[0]);
+        each_pair<L>([&](auto k) {
+            TLBM_ROUND_EACH
+            constexpr int s = k, b = L::bb[s];
+            const T w2 = T(2.0) * w[s];
+            n[s] = fma_t(-w2, m0, n[s]);
+            n[b] = fma_t(-w2, edot<T>(L::ex[s], L::ey[s], L::ez[s], cx, cy, cz), n[b]);
+        });
+    }
+    if (ends) pairs_rebuild<L, T, SC>(f, n, inlet, outlet, h, Ux, Uy, Uz, w);
+    if (uy_head && __any(t == 5)) {
+        // set_uz_bc (LatticeStructure.hpp:166-177); the y term reads uy of
+        // node s of this step, as the reference's uy[spd] does
+        const T ubc = a.inlet_uz ? T(a.inlet_uz[g % a.nxny]) : num<T>(a.u_bc, a.fl.u_bc);
+        const T ux = mx * inv, uz = mz * inv, r3 = t == 5 ? T(3.0) * rho : T(0.0);
+        each_pair<L>([&](auto k) {
+            constexpr int s = k, b = L::bb[s];
+            T in[2];
+            each<0, 2>([&](auto i) {
+                constexpr int d = i ? b : s;
+                T br = T(-0.0);
+                if (L::ez[d] > 0) br += (ubc - uz); else if (L::ez[d] < 0) br -= (ubc - uz);
+                if (L::ex[d] > 0) br -= ux; else if (L::ex[d] < 0) br += ux;
+                if (L::ey[d] > 0) br -= uy_head[d]; else if (L::ey[d] < 0) br += uy_head[d];
+                in[i] = (SC ? r3 : r3 * w[s]) * br;
+                f[d] += in[i];
+            });
+            n[s] += in[0] + in[1];
+            n[b] += in[0] - in[1];
+        });
+    }
+}
+
+// Pi of a node from the pair sums of n[] (see node_stress).
+template <class L, class T, bool SC>
+__device__ inline void pair_stress(const T (&n)[L::Q], T (&pi)[6], const T (&w)[L::Q]) {
+#pragma unroll
+    for (int k = 0; k < 6; ++k) pi[k] = T(-0.0);
+    each_pair<L>([&](auto k) {
+        constexpr int s = k;
+        const T v = SC ? n[s] * w[s] : n[s];
+        if (L::ex[s] != 0) pi[0] += v;
+        if (L::ey[s] != 0) pi[1] += v;
+        if (L::ez[s] != 0) pi[2] += v;
+        if (L::ex[s] * L::ey[s] > 0) pi[3] += v; else if (L::ex[s] * L::ey[s] < 0) pi[3] -= v;
+        if (L::ex[s] * L::ez[s] > 0) pi[4] += v; else if (L::ex[s] * L::ez[s] < 0) pi[4] -= v;
+        if (L::ey[s] * L::ez[s] > 0) pi[5] += v; else if (L::ey[s] * L::ez[s] < 0) pi[5] -= v;
+    });
+}
+
+// Relaxation from n[] at rate om, and the solid node's whole-vector
+// bounce-back without relaxation (TLBM_Partition.cpp:750-756,
+// D3Q19LatticeStructure.hpp:65-76): rate 0, and the pairs trade places.
+// solids: the wavefront's solid lanes, __ballot(t == 1) (scalar registers, so
+// that the node type need not stay in a vector register until here).
+template <class L, class T>
+__device__ inline void pairs_relax(T (&f)[L::Q], const T (&n)[L::Q], uint64_t solids, T om, const StepArgs &a) {
+    const bool solid = __builtin_amdgcn_inverse_ballot_w64(solids);
+    om = solid || a.dynamics != 1 ? T(0.0) : om;
+    const T half = T(-0.5) * om;
+    f[0] = fma_t(-om, n[0], f[0]);
+    each_pair<L>([&](auto k) {
+        constexpr int s = k, b = L::bb[s];
+        f[s] = fma_t(half, n[s] + n[b], f[s]);
+        f[b] = fma_t(half, n[s] - n[b], f[b]);
+    });
+    if (solids) {
+        each_pair<L>([&](auto k) {
+            constexpr int s = k, b = L::bb[s];
+            const T x = f[s];
+            f[s] = solid ? f[b] : x;
+            f[b] = solid ? x : f[b];
+        });
+    }
+}
 
 // The whole reference update of one node (TLBM_Partition.cpp:742-807).
 // CONSERVE: fluid nodes relax with node_relax_conserving.  SC: the scaled
@@ -803,24 +1079,28 @@ __device__ inline void node_update(T (&f)[L::Q], int t, T &rho, T &ux, T &uy, T 
                                    const StepArgs &a, const T *__restrict__ uy_head,
                                    const T (&w)[L::Q], uint32_t g) {
     static_assert(!(SC && CONSERVE), "the conserving relax works on d");
+    if constexpr (COLLIDE && SHIFT) {
+        T n[L::Q], om = num<T>(a.omega, a.fl.omega);
+        const uint64_t solids = __ballot(t == 1);
+        pairs_prepare<L, T, SC, CONSERVE>(f, n, t, a, uy_head, w, g);
+        if (a.smag) {
+            T pi[6];
+            pair_stress<L, T, SC>(n, pi, w);
+            om = smagorinsky_omega<T, SC>(pi, a);
+        }
+        pairs_relax<L, T>(f, n, solids, om, a);
+        return;
+    }
     T feq[L::Q];
     if (!node_prepare<L, T, SHIFT, COLLIDE, SC>(f, feq, t, rho, ux, uy, uz, a, uy_head, w, g)) return;
     if (!COLLIDE) return;
-    T om = T(a.omega);
+    T om = num<T>(a.omega, a.fl.omega);
     if (a.smag) {
         T pi[6];
         node_stress<L, T, SC>(f, feq, pi, w);
         om = smagorinsky_omega<T, SC>(pi, a);
     }
-    if (a.dynamics == 1) {
-        if constexpr (CONSERVE) {
-            if (t == 0) {
-                node_relax_conserving<L>(f, feq, w, om, rho, ux, uy, uz, a);
-                return;
-            }
-        }
-        node_relax<L, T>(f, feq, om);
-    }
+    if (a.dynamics == 1) node_relax<L, T>(f, feq, om);
 }
 
 // Has the step kernels' prologue load, in one batch of scalar loads, the
@@ -852,6 +1132,8 @@ __device__ inline void load_args_early(const StepArgs &a, const void *fin) {
 template <class L, int ST, int MODE, bool REMAP = true, bool NTLOAD = false, bool NTSTORE = true,
           int BS = kBlock>
 __global__ void __launch_bounds__(BS)
+__attribute__((amdgpu_waves_per_eu(MODE == MODE_STEP ? kStepWaves<ST, L::Q> : 1,
+                                   MODE == MODE_STEP ? kStepWavesMax<ST, L::Q> : 8)))
 k_lbm(const typename StorageT<ST>::st *__restrict__ fin, typename StorageT<ST>::st *__restrict__ fout,
       const uint8_t *__restrict__ nd_type, const uint8_t *__restrict__ chunk_type,
       void *__restrict__ out, const typename StorageT<ST>::T *__restrict__ uy_head, StepArgs a) {
@@ -881,26 +1163,22 @@ k_lbm(const typename StorageT<ST>::st *__restrict__ fin, typename StorageT<ST>::
     if (MODE == MODE_STEP && a.row_chunks && pull_rel_ok<BS>(blk * BS, a)) {
         PullRow<L, ST> pr;
         pr.init(fin, blk * BS, x, y, g - r, a);
-#pragma unroll
-        for (int s = 0; s < Q; ++s) f[s] = S::in(pr.template load<NTLOAD>(s, L::ex[s], L::ey[s], L::ez[s]), s, a);
+        each<0, Q>([&](auto s) { f[s] = S::in(pr.template load<NTLOAD>(s, L::ex[s], L::ey[s], L::ez[s]), s, a); });
     } else if (MODE == MODE_STEP && pull_rel_ok<BS>(blk * BS, a)) {
         PullRel<L, ST> pr;
         pr.init(fin, blk * BS, x, y, g - r, a);
-#pragma unroll
-        for (int s = 0; s < Q; ++s) f[s] = S::in(pr.template load<NTLOAD>(s, L::ex[s], L::ey[s], L::ez[s]), s, a);
+        each<0, Q>([&](auto s) { f[s] = S::in(pr.template load<NTLOAD>(s, L::ex[s], L::ey[s], L::ez[s]), s, a); });
     } else {
         Gather gat;
         gat.init(x, y, z, a);
-#pragma unroll
-        for (int s = 0; s < Q; ++s) {
+        each<0, Q>([&](auto s) {
             const st *p = fin + fidx<Q>(s, gat.src(L::ex[s], L::ey[s], L::ez[s]), a);
             f[s] = S::in(NTLOAD ? __builtin_nontemporal_load(p) : *p, s, a);
-        }
+        });
     }
     if constexpr (MODE == MODE_STEP && kGatherPrio<ST, Q>) __builtin_amdgcn_s_setprio(0);
     T w[Q];
-#pragma unroll
-    for (int s = 0; s < Q; ++s) w[s] = S::weight(s, a);
+    each<0, Q>([&](auto s) { w[s] = S::weight(weight_class<L>(s), a); });
     if constexpr (!kTypeAhead<ST>) t0 = type_first<MODE>(nd_type, chunk_type, chunk, g);
     const int t = type_final<MODE>(t0, nd_type, chunk_type, g);
     T rho, ux, uy, uz;
@@ -909,9 +1187,7 @@ k_lbm(const typename StorageT<ST>::st *__restrict__ fin, typename StorageT<ST>::
                                                                          uy_head, w, g);
         const PushOut<L, ST> po(fout, (blk * BS) >> StorageT<ST>::kCB, g);
         const uint32_t rs = ST == ST_F16 ? round_stream(g, a.step) : 0u;
-#pragma unroll
-        for (int s = 0; s < Q; ++s)
-            po.template store<NTSTORE>(s, S::step_out(f[s], s, a, rs + uint32_t(s) * kStreamStep));
+        each<0, Q>([&](auto s) { po.template store<NTSTORE>(s, S::step_out(f[s], s, a, rs + uint32_t(s) * kStreamStep)); });
     } else if (MODE == MODE_STRESS) {
         T feq[Q], pi[6] = {T(0), T(0), T(0), T(0), T(0), T(0)};
         T c = T(0);
@@ -919,7 +1195,7 @@ k_lbm(const typename StorageT<ST>::st *__restrict__ fin, typename StorageT<ST>::
                                                             w, g) &&
             a.dynamics == 1) {
             node_stress<L, T, S::kScaled>(f, feq, pi, w);
-            const T om = a.smag ? smagorinsky_omega<T>(pi, a) : T(a.omega);
+            const T om = a.smag ? smagorinsky_omega<T>(pi, a) : num<T>(a.omega, a.fl.omega);
             c = T(0.5) * om - T(1);
         }
         T *macro = static_cast<T *>(out);
@@ -949,6 +1225,47 @@ k_lbm(const typename StorageT<ST>::st *__restrict__ fin, typename StorageT<ST>::
     }
 }
 
+// The update of a node whose relaxation time is the network's (mlp.h).  Every
+// lane of the wavefront takes part.  ready() is called once before the network
+// reads m (the workgroup's copy of the weights).  A solid node's result is
+// not used.
+template <class L, int ST, class F>
+__device__ inline void network_update(float (&f)[L::Q], int t, const StepArgs &a, const float *__restrict__ uy_head,
+                                      const float (&w)[L::Q], uint32_t g, const MlpPacked *m, F ready) {
+    using S = StorageT<ST>;
+    float n[L::Q], pi[6];
+    const uint64_t solids = __ballot(t == 1);
+    pairs_prepare<L, float, S::kScaled, kConserve<ST, L::Q>>(f, n, t, a, uy_head, w, g);
+    // formed here, not sunk past the network with its three operands (registers)
+    __asm__ volatile("" : "+v"(n[0]));
+    pair_stress<L, float, S::kScaled>(n, pi, w);
+    float feat[kMlpIn];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) feat[k] = pi[k] * a.cl_in;
+    // the norm feature is rounded to bf16: the hardware square root (1 ulp) suffices
+    feat[6] = __builtin_amdgcn_sqrtf(pi[0] * pi[0] + pi[1] * pi[1] + pi[2] * pi[2] +
+                                     2.0f * (pi[3] * pi[3] + pi[4] * pi[4] + pi[5] * pi[5])) *
+              a.cl_in;
+    ready();
+    const float zz = mlp_wave(feat, m);
+    const float om = __builtin_amdgcn_rcpf(a.tau0 + a.cl_out * softplus_f(zz));  // 1 ulp
+    pairs_relax<L, float>(f, n, solids, om, a);
+}
+
+// This thread's share of copying the network's weights to LDS, by direct
+// global-to-LDS loads (lane i of a wavefront writes 16 bytes at the
+// wavefront's LDS base + 16 i).
+__device__ inline void stage_network(const MlpPacked *src, MlpPacked *dst) {
+    using gptr = const __attribute__((address_space(1))) void *;
+    using lptr = __attribute__((address_space(3))) void *;
+    static_assert(sizeof(MlpPacked) % 16 == 0, "16-byte loads");
+    if (threadIdx.x < sizeof(MlpPacked) / 16) {
+        const uint32_t wave_base = (threadIdx.x & ~63u) * 16;  // uniform per wavefront
+        __builtin_amdgcn_global_load_lds((gptr)(reinterpret_cast<const char *>(src) + threadIdx.x * 16),
+                                         (lptr)(reinterpret_cast<char *>(dst) + wave_base), 16, 0, 0);
+    }
+}
+
 // Step with the learned closure in place of Smagorinsky (FP32/FP16 storage).
 // One node per lane as k_lbm; every lane of a wavefront runs the network
 // together (lanes past the last node work on the last node and store
@@ -962,25 +1279,17 @@ k_lbm_closure(const typename StorageT<ST>::st *__restrict__ fin, typename Storag
     using T = typename S::T;
     using st = typename S::st;
     constexpr int Q = L::Q;
-    // The network's packed weights, staged once per workgroup by direct
-    // global-to-LDS loads (global_load_lds_dwordx4: lane i of a wavefront
-    // writes 16 bytes at the wavefront's LDS base + 16 i).  They go out ahead
-    // of the gathers and hold no registers; a load into registers followed by
-    // an LDS write made every wavefront wait one L2 round trip before issuing
-    // its gathers (FP16 D3Q19 128x128x512: 147 -> 143 us per step; FP32
-    // 217 -> 207).  A copy per wavefront, which needs no workgroup barrier,
-    // was slower (148 us).
+    // The network's packed weights, staged once per workgroup.  The loads go
+    // out ahead of the gathers and hold no registers; a load into registers
+    // followed by an LDS write made every wavefront wait one L2 round trip
+    // before issuing its gathers (FP16 D3Q19 128x128x512: 147 -> 143 us per
+    // step; FP32 217 -> 207).  A copy per wavefront, which needs no workgroup
+    // barrier, was slower (148 us).
     load_args_early(a, fin);
     __asm__ volatile("" ::"s"(a.mlp));  // in the same batch
     __shared__ MlpPacked smlp;
-    static_assert(sizeof(MlpPacked) % 16 == 0 && sizeof(MlpPacked) <= 16u * BS, "one 16-byte load per lane");
-    if (threadIdx.x < sizeof(MlpPacked) / 16) {
-        using gptr = const __attribute__((address_space(1))) void *;
-        using lptr = __attribute__((address_space(3))) void *;
-        const uint32_t wave_base = (threadIdx.x & ~63u) * 16;  // uniform per wavefront
-        __builtin_amdgcn_global_load_lds((gptr)(reinterpret_cast<const char *>(a.mlp) + threadIdx.x * 16),
-                                         (lptr)(reinterpret_cast<char *>(&smlp) + wave_base), 16, 0, 0);
-    }
+    static_assert(sizeof(MlpPacked) <= 16u * BS, "one 16-byte load per lane");
+    stage_network(a.mlp, &smlp);
     const uint32_t g0 = blockIdx.x * BS + threadIdx.x;
     const bool live = g0 < a.N;
     const uint32_t g = live ? g0 : a.N - 1;
@@ -994,57 +1303,30 @@ k_lbm_closure(const typename StorageT<ST>::st *__restrict__ fin, typename Storag
     if (a.row_chunks && pull_rel_ok<BS>(blockIdx.x * BS, a)) {
         PullRow<L, ST> pr;
         pr.init(fin, blockIdx.x * BS, x, y, g - r, a);
-#pragma unroll
-        for (int s = 0; s < Q; ++s) f[s] = S::in(pr.template load<NTLOAD>(s, L::ex[s], L::ey[s], L::ez[s]), s, a);
+        each<0, Q>([&](auto s) { f[s] = S::in(pr.template load<NTLOAD>(s, L::ex[s], L::ey[s], L::ez[s]), s, a); });
     } else if (pull_rel_ok<BS>(blockIdx.x * BS, a)) {
         PullRel<L, ST> pr;
         pr.init(fin, blockIdx.x * BS, x, y, g - r, a);
-#pragma unroll
-        for (int s = 0; s < Q; ++s) f[s] = S::in(pr.template load<NTLOAD>(s, L::ex[s], L::ey[s], L::ez[s]), s, a);
+        each<0, Q>([&](auto s) { f[s] = S::in(pr.template load<NTLOAD>(s, L::ex[s], L::ey[s], L::ez[s]), s, a); });
     } else {
         Gather gat;
         gat.init(x, y, z, a);
-#pragma unroll
-        for (int s = 0; s < Q; ++s) {
+        each<0, Q>([&](auto s) {
             const st *p = fin + fidx<Q>(s, gat.src(L::ex[s], L::ey[s], L::ez[s]), a);
             f[s] = S::in(NTLOAD ? __builtin_nontemporal_load(p) : *p, s, a);
-        }
+        });
     }
     T w[Q];
-#pragma unroll
-    for (int s = 0; s < Q; ++s) w[s] = S::weight(s, a);
+    each<0, Q>([&](auto s) { w[s] = S::weight(weight_class<L>(s), a); });
     const int t = type_final<MODE_STEP>(t0, nd_type, chunk_type, g);
-    T feq[Q], rho, ux, uy, uz;
-    const bool relaxes = node_prepare<L, T, S::kShift, true, S::kScaled>(f, feq, t, rho, ux, uy, uz,
-                                                                         a, uy_head, w, g);
-    T pi[6];
-    node_stress<L, T, S::kScaled>(f, feq, pi, w);
-    float feat[kMlpIn];
-#pragma unroll
-    for (int k = 0; k < 6; ++k) feat[k] = float(pi[k]) * a.cl_in;
-    // the norm feature is rounded to bf16: the hardware square root (1 ulp) suffices
-    feat[6] = __builtin_amdgcn_sqrtf(float(pi[0] * pi[0] + pi[1] * pi[1] + pi[2] * pi[2] +
-                                           T(2) * (pi[3] * pi[3] + pi[4] * pi[4] + pi[5] * pi[5]))) *
-              a.cl_in;
-
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wavefront's load into smlp has landed
-    __syncthreads();                     // smlp complete (every lane of the workgroup gets here)
-    const float zz = mlp_wave(feat, &smlp);
-    const float om = __builtin_amdgcn_rcpf(a.tau0 + a.cl_out * softplus_f(zz));  // 1 ulp
-    if (a.dynamics == 1) {
-        if (kConserve<ST, Q> && t == 0)
-            node_relax_conserving<L>(f, feq, w, om, rho, ux, uy, uz, a);
-        else
-            // the one node type that does not relax, the solid node, has
-            // feq = f, so the rate 0 leaves it exactly as it is; no branch
-            node_relax<L, T>(f, feq, relaxes ? T(om) : T(0));
-    }
+    network_update<L, ST>(f, t, a, uy_head, w, g, &smlp, [] {
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wavefront's load into smlp has landed
+        __syncthreads();                     // smlp complete (every lane of the workgroup gets here)
+    });
     if (!live) return;
     const PushOut<L, ST> po(fout, (blockIdx.x * BS) >> StorageT<ST>::kCB, g);
     const uint32_t rs = ST == ST_F16 ? round_stream(g, a.step) : 0u;
-#pragma unroll
-    for (int s = 0; s < Q; ++s)
-        po.template store<true>(s, S::step_out(f[s], s, a, rs + uint32_t(s) * kStreamStep));
+    each<0, Q>([&](auto s) { po.template store<true>(s, S::step_out(f[s], s, a, rs + uint32_t(s) * kStreamStep)); });
 }
 
 }  // namespace tlbm

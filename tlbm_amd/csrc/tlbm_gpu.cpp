@@ -272,6 +272,14 @@ int tlbm_gpu_create(const tlbm_params *p, const uint8_t *nd_type, tlbm_gpu **out
     a.rho_bc = p->rho_lbm;
     a.inv_1mu = 1. / (1. - p->u_lbm);
     a.inv_rho_bc = 1. / p->rho_lbm;
+    a.fl.cs = float(a.cs);
+    a.fl.omega = float(a.omega);
+    a.fl.nu = float(a.nu);
+    a.fl.nu2 = float(a.nu2);
+    a.fl.u_bc = float(a.u_bc);
+    a.fl.rho_bc = float(a.rho_bc);
+    a.fl.inv_1mu = float(a.inv_1mu);
+    a.fl.inv_rho_bc = float(a.inv_rho_bc);
     a.cb = chunk_bits(storage_bytes(p->storage));
     a.div_nx = tlbm::udiv_magic(a.nx);
     a.div_nxny = tlbm::udiv_magic(a.nxny);
