@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "launch.h"
+#include "pair_plan.h"
 
 namespace {
 thread_local std::string g_err;
@@ -165,6 +166,9 @@ struct tlbm_gpu {
     float *inlet = nullptr;            // nx*ny inlet u_z profile
     double *avg = nullptr;             // 4*N FP64 time-average sums
     bool avg_on = false;
+    // steps may go two at a time (lbm_pair.h): without and with the network
+    bool pair[2] = {false, false};
+    tlbm::PairPlan plan[2] = {};
     int64_t avg_steps = 0;
 };
 
@@ -309,6 +313,18 @@ int tlbm_gpu_create(const tlbm_params *p, const uint8_t *nd_type, tlbm_gpu **out
         return code;
     };
     if (int rc = fixed_partials(&h->fixed_partial)) return cleanup_fail(rc);
+    {
+        int dev = 0, cus = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+            cus = 0;
+        for (int net = 0; net < 2; ++net)
+            h->pair[net] = !has_lid && cus > 0 && (net == 0 || p->storage == TLBM_STORAGE_F32) &&
+                           tlbm::pair_plan(
+                               a.nx, a.ny, a.nz, Q, int(storage_bytes(p->storage)), net != 0, uint32_t(cus),
+                               [&](int k, tlbm::PairShape &s) { return h->ops->pair_shape(Q, k, s); },
+                               &h->plan[net]);
+    }
     hipError_t e;
     if ((e = hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking)) != hipSuccess)
         return cleanup_fail(fail(TLBM_EHIP, std::string("hipStreamCreate: ") + hipGetErrorString(e)));
@@ -385,7 +401,23 @@ int tlbm_gpu_destroy(tlbm_gpu *h) {
 }
 
 static int queue_steps(tlbm_gpu *h, int nsteps) {
-    for (int k = 0; k < nsteps; ++k) {
+    int k = 0;
+    // Two steps at a time, except the call's last one (or two): the state the
+    // last step reads stays in f[1 - cur] for the moments, the residual and
+    // the box filter.
+    const int net = h->args.closure ? 1 : 0;
+    if (h->pair[net] && !h->avg_on) {
+        for (; k + 2 < nsteps; k += 2) {
+            h->args.step = uint32_t(h->step_count);
+            hipError_t e = h->ops->lbm_pair(h->Q, h->f[h->cur], h->f[1 - h->cur], h->nd, h->plan[net], h->args,
+                                            h->stream);
+            if (e != hipSuccess) return fail(TLBM_EHIP, std::string("two steps: ") + hipGetErrorString(e));
+            h->cur = 1 - h->cur;
+            h->step_count += 2;
+            h->steps_since_set += 2;
+        }
+    }
+    for (; k < nsteps; ++k) {
         const void *fin = h->f[h->cur];
         void *fout = h->f[1 - h->cur];
         if (h->has_lid) {
