@@ -2,11 +2,10 @@
 // (mlp.h), and their C-ABI (include/tlbm_gpu.h, tlbm_mlp_*).
 //
 // Training: each step draws `batch` samples (a counter-based hash of seed,
-// step and position picks each index), one thread per sample computes the
-// forward and backward pass in FP32 with the parameters in LDS, and the
-// workgroup turns its 128 samples' activations and deltas into the weight
-// gradient as small LDS matrix products.  Per-workgroup partial gradients
-// are folded in a fixed order by a second kernel, which applies Adam.
+// step and position picks each index).  A wavefront takes 32 samples at a
+// time through the forward and the backward pass and their weight gradient
+// with FP32 MFMA and keeps the gradient in registers; per-workgroup partial
+// gradients are folded in a fixed order by a second kernel, which applies Adam.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -19,15 +18,13 @@
 
 namespace tlbm {
 
-constexpr int kTB = 128;            // samples per training workgroup
+constexpr int kUnit = 32;           // samples a wavefront takes at a time
+constexpr int kGradWaves = 4;       // wavefronts of a training workgroup
+constexpr int kGradBlocks = 256;    // at most one training workgroup per CU
 constexpr int kGradLen = kMlpParams + 1;  // + loss
-
-struct ParamView {
-    const float *W1, *b1, *W2, *b2, *w3, *b3;
-    __device__ ParamView(const float *p)
-        : W1(p), b1(p + kMlpH * kMlpIn), W2(b1 + kMlpH), b2(W2 + kMlpH * kMlpH), w3(b2 + kMlpH),
-          b3(w3 + kMlpH) {}
-};
+// offsets of the flat parameters
+constexpr int kB1 = kMlpH * kMlpIn, kW2 = kB1 + kMlpH, kB2 = kW2 + kMlpH * kMlpH, kW3 = kB2 + kMlpH,
+              kB3 = kW3 + kMlpH;
 
 __device__ inline uint64_t mix64(uint64_t x) {  // splitmix64 finaliser
     x += 0x9e3779b97f4a7c15ull;
@@ -36,139 +33,201 @@ __device__ inline uint64_t mix64(uint64_t x) {  // splitmix64 finaliser
     return x ^ (x >> 31);
 }
 
-// mode 0: sample i of the batch is index first + i; mode 1: a hashed index.
-__global__ void __launch_bounds__(kTB)
+// Partial gradient of one workgroup's samples.  mode 0: sample i of the batch
+// is index first + i; mode 1: a hashed index.
+//
+// All five products are v_mfma_f32_32x32x2_f32 (lane l supplies A[l%32][g] and
+// B[g][l%32], g = l/32; lane l holds, in register 4q + r, row 8q + 4g + r of
+// column l%32).  With the samples as columns a layer's output registers are
+// the next product's B operand: K step (q, r) takes units 8q + r and
+// 8q + 4 + r, and the weights are held per lane in that order, W2 both as it
+// is (forward) and transposed (backward).  The weight gradients contract over
+// the samples, so activations and deltas pass through LDS, written by rows of
+// a sample and read by columns, within the wavefront.  b1 is the weight of an
+// eighth input 1, so its gradient is that of W1.
+//
+// Bound by the MFMA rate: 68 products of 64 cycles per 32 samples, 3.6 us for
+// 65536 samples.  One thread per sample with the weights in LDS took 46 us
+// (an LDS read per multiply-add), and a fold by one thread per parameter
+// 159 us (512 dependent loads).
+__global__ void __launch_bounds__(kGradWaves * 64)
 k_mlp_grad(const float *__restrict__ X, const float *__restrict__ Tg, int64_t M, int64_t first,
            int mode, uint64_t seed, int64_t step, int64_t batch, const float *__restrict__ params,
            float *__restrict__ partial) {
-    __shared__ float sp[kMlpParams];
-    __shared__ float sa[kTB][kMlpH + 1];
-    __shared__ float sb[kTB][kMlpH + 1];
-    __shared__ float sred[kTB];
-    for (int k = threadIdx.x; k < kMlpParams; k += kTB) sp[k] = params[k];
-    __syncthreads();
-    const ParamView P(sp);
-    const int tid = threadIdx.x;
-    const int64_t pos = int64_t(blockIdx.x) * kTB + tid;
-    const bool live = pos < batch;
-    int64_t idx = 0;
-    if (live) idx = mode == 0 ? first + pos : int64_t(mix64(seed ^ mix64(uint64_t(step) * 0x100000001ull + uint64_t(pos))) % uint64_t(M));
-    float x[kMlpIn], h1[kMlpH], h2[kMlpH];
+    constexpr int S = kMlpH + 4;  // row of a sample in LDS: 16-byte aligned, banks spread
+    struct Wave {
+        float d[kUnit * S];   // deltas by sample (d2, then d1)
+        float h[kUnit * S];   // h1 by sample
+        float x[kUnit * 12];  // inputs by sample
+    };
+    __shared__ alignas(16) Wave sw[kGradWaves];
+    __shared__ float sum[kGradLen];
+    const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, c = l & 31, g = l >> 5;
+    Wave &W = sw[wave];
+    const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    // operands that stay: W1 with b1 as input 7, W2, its transpose, b2 and w3
+    float a1[4], a2[16], a2t[16], w3[16];
+    f32x16 b2;
 #pragma unroll
-    for (int i = 0; i < kMlpIn; ++i) x[i] = live ? X[idx * kMlpIn + i] : 0.f;
-#pragma unroll
-    for (int j = 0; j < kMlpH; ++j) {
-        float a = P.b1[j];
-#pragma unroll
-        for (int i = 0; i < kMlpIn; ++i) a += P.W1[j * kMlpIn + i] * x[i];
-        h1[j] = fmaxf(a, 0.f);
+    for (int t = 0; t < 4; ++t) {
+        const int k = 2 * t + g;
+        a1[t] = k < kMlpIn ? params[c * kMlpIn + k] : params[kB1 + c];
     }
 #pragma unroll
-    for (int j = 0; j < kMlpH; ++j) {
-        float a = P.b2[j];
-#pragma unroll
-        for (int i = 0; i < kMlpH; ++i) a += P.W2[j * kMlpH + i] * h1[i];
-        h2[j] = fmaxf(a, 0.f);
+    for (int k = 0; k < 16; ++k) {
+        const int u = 8 * (k >> 2) + 4 * g + (k & 3);
+        a2[k] = params[kW2 + c * kMlpH + u];
+        a2t[k] = params[kW2 + u * kMlpH + c];
+        b2[k] = params[kB2 + u];
+        w3[k] = params[kW3 + u];
     }
-    float z = P.b3[0];
+    const float b3 = params[kB3];
+    f32x16 gW2 = zero, gW1 = zero, gb2 = zero, gw3 = zero;
+    float gb3 = 0.f, loss = 0.f;
+    const int64_t units = (batch + kUnit - 1) / kUnit, stride = int64_t(gridDim.x) * kGradWaves;
+    for (int64_t un = int64_t(blockIdx.x) * kGradWaves + wave; un < units; un += stride) {
+        const int64_t pos = un * kUnit + c;
+        const bool live = pos < batch;
+        int64_t idx = 0;
+        if (live)
+            idx = mode == 0 ? first + pos
+                            : int64_t(mix64(seed ^ mix64(uint64_t(step) * 0x100000001ull + uint64_t(pos))) % uint64_t(M));
+        float x[4];
 #pragma unroll
-    for (int j = 0; j < kMlpH; ++j) z += P.w3[j] * h2[j];
-    const float y = z > 20.f ? z : log1pf(expf(z));
-    const float r = live ? y - Tg[idx] : 0.f;
-    const float loss = 0.5f * r * r;
-    const float dz = r / (1.f + expf(-z)) / float(batch);
-    float d2[kMlpH];
+        for (int t = 0; t < 4; ++t) {
+            const int k = 2 * t + g;
+            x[t] = k == kMlpIn ? 1.f : live ? X[idx * kMlpIn + k] : 0.f;
+        }
+        const float target = live ? Tg[idx] : 0.f;
+        f32x16 h1 = zero;
 #pragma unroll
-    for (int j = 0; j < kMlpH; ++j) d2[j] = h2[j] > 0.f ? dz * P.w3[j] : 0.f;
-    // phase A: dW2 = sum_s d2 h1^T, db2
+        for (int t = 0; t < 4; ++t) h1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[t], x[t], h1, 0, 0, 0);
 #pragma unroll
-    for (int j = 0; j < kMlpH; ++j) {
-        sa[tid][j] = h1[j];
-        sb[tid][j] = d2[j];
+        for (int k = 0; k < 16; ++k) h1[k] = fmaxf(h1[k], 0.f);
+        f32x16 h2 = b2;
+#pragma unroll
+        for (int k = 0; k < 16; ++k) h2 = __builtin_amdgcn_mfma_f32_32x32x2f32(a2[k], h1[k], h2, 0, 0, 0);
+        float z = 0.f;
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            h2[k] = fmaxf(h2[k], 0.f);
+            z += w3[k] * h2[k];
+        }
+        z = (z + __shfl_xor(z, 32, 64)) + b3;
+        const float y = z > 20.f ? z : log1pf(expf(z));
+        const float r = live ? y - target : 0.f;
+        const float dz = r / (1.f + expf(-z)) / float(batch);
+        if (g == 0) {
+            loss += 0.5f * r * r;
+            gb3 += dz;
+        }
+        f32x16 d2;
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            d2[k] = h2[k] > 0.f ? dz * w3[k] : 0.f;
+            gb2[k] += d2[k];
+            gw3[k] += dz * h2[k];
+        }
+        f32x16 d1 = zero;
+#pragma unroll
+        for (int k = 0; k < 16; ++k) d1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a2t[k], d2[k], d1, 0, 0, 0);
+        // dW2 = sum_s d2 h1^T
+        typedef float f32x4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            *reinterpret_cast<f32x4 *>(&W.d[c * S + 8 * q + 4 * g]) = f32x4{d2[4 * q], d2[4 * q + 1], d2[4 * q + 2], d2[4 * q + 3]};
+            *reinterpret_cast<f32x4 *>(&W.h[c * S + 8 * q + 4 * g]) = f32x4{h1[4 * q], h1[4 * q + 1], h1[4 * q + 2], h1[4 * q + 3]};
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t) W.x[c * 12 + 2 * t + g] = x[t];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+        for (int k = 0; k < 16; ++k)
+            gW2 = __builtin_amdgcn_mfma_f32_32x32x2f32(W.d[(2 * k + g) * S + c], W.h[(2 * k + g) * S + c], gW2, 0, 0, 0);
+        // dW1 = sum_s d1 x^T
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            f32x4 v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = h1[4 * q + e] > 0.f ? d1[4 * q + e] : 0.f;
+            *reinterpret_cast<f32x4 *>(&W.d[c * S + 8 * q + 4 * g]) = v;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            const float xv = c < 8 ? W.x[(2 * k + g) * 12 + (c & 7)] : 0.f;
+            gW1 = __builtin_amdgcn_mfma_f32_32x32x2f32(W.d[(2 * k + g) * S + c], xv, gW1, 0, 0, 0);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
-    __syncthreads();
+    // sums over the samples' lanes: db2 and dw3 unit by unit through LDS
+    // (row k of 64 lanes in W.d and W.h), db3 and the loss by exchange
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        W.d[k * 64 + l] = gb2[k];
+        W.h[k * 64 + l] = gw3[k];
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        gb3 += __shfl_xor(gb3, off, 64);
+        loss += __shfl_xor(loss, off, 64);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    float unit = 0.f;  // lanes 0-31: db2 of unit c; lanes 32-63: dw3
+    {
+        const float *src = (g == 0 ? W.d : W.h) + (4 * (c >> 3) + (c & 3)) * 64 + 32 * ((c >> 2) & 1);
+        for (int k = 0; k < 32; ++k) unit += src[(k + c) & 31];
+    }
+    // the wavefronts' sums, in order
+    for (int v = 0; v < kGradWaves; ++v) {
+        if (wave == v) {
+            auto add = [&](int at, float val) { sum[at] = v == 0 ? val : sum[at] + val; };
+#pragma unroll
+            for (int k = 0; k < 16; ++k) {
+                const int u = 8 * (k >> 2) + 4 * g + (k & 3);
+                add(kW2 + u * kMlpH + c, gW2[k]);
+                if (c < kMlpIn) add(u * kMlpIn + c, gW1[k]);
+                if (c == kMlpIn) add(kB1 + u, gW1[k]);
+            }
+            add((g == 0 ? kB2 : kW3) + c, unit);
+            if (l == 0) add(kB3, gb3);
+            if (l == 1) add(kMlpParams, loss);
+        }
+        __syncthreads();
+    }
     float *out = partial + size_t(blockIdx.x) * kGradLen;
-    float *gW1 = out, *gb1 = gW1 + kMlpH * kMlpIn, *gW2 = gb1 + kMlpH, *gb2 = gW2 + kMlpH * kMlpH,
-          *gw3 = gb2 + kMlpH, *gb3 = gw3 + kMlpH;
-    for (int e = tid; e < kMlpH * kMlpH; e += kTB) {
-        const int j = e / kMlpH, i = e % kMlpH;
-        float acc = 0.f;
-        for (int s = 0; s < kTB; ++s) acc += sb[s][j] * sa[s][i];
-        gW2[e] = acc;
-    }
-    if (tid < kMlpH) {
-        float acc = 0.f;
-        for (int s = 0; s < kTB; ++s) acc += sb[s][tid];
-        gb2[tid] = acc;
-    }
-    // d1 = (W2^T d2) masked by h1 > 0
-    float d1[kMlpH];
-#pragma unroll
-    for (int i = 0; i < kMlpH; ++i) {
-        float a = 0.f;
-#pragma unroll
-        for (int j = 0; j < kMlpH; ++j) a += P.W2[j * kMlpH + i] * d2[j];
-        d1[i] = h1[i] > 0.f ? a : 0.f;
-    }
-    __syncthreads();
-    // phase B: dW1 = sum_s d1 x^T, db1
-#pragma unroll
-    for (int j = 0; j < kMlpH; ++j) sa[tid][j] = d1[j];
-#pragma unroll
-    for (int i = 0; i < kMlpIn; ++i) sb[tid][i] = x[i];
-    __syncthreads();
-    for (int e = tid; e < kMlpH * kMlpIn; e += kTB) {
-        const int j = e / kMlpIn, i = e % kMlpIn;
-        float acc = 0.f;
-        for (int s = 0; s < kTB; ++s) acc += sa[s][j] * sb[s][i];
-        gW1[e] = acc;
-    }
-    if (tid < kMlpH) {
-        float acc = 0.f;
-        for (int s = 0; s < kTB; ++s) acc += sa[s][tid];
-        gb1[tid] = acc;
-    }
-    __syncthreads();
-    // phase C: dw3 = sum_s dz h2, db3, loss
-#pragma unroll
-    for (int j = 0; j < kMlpH; ++j) sa[tid][j] = h2[j];
-    sb[tid][0] = dz;
-    sred[tid] = loss;
-    __syncthreads();
-    if (tid < kMlpH) {
-        float acc = 0.f;
-        for (int s = 0; s < kTB; ++s) acc += sb[s][0] * sa[s][tid];
-        gw3[tid] = acc;
-    }
-    if (tid == kMlpH) {
-        float acc = 0.f;
-        for (int s = 0; s < kTB; ++s) acc += sb[s][0];
-        gb3[0] = acc;
-    }
-    if (tid == kMlpH + 1) {
-        float acc = 0.f;
-        for (int s = 0; s < kTB; ++s) acc += sred[s];
-        out[kMlpParams] = acc;
-    }
+    for (int k = threadIdx.x; k < kGradLen; k += kGradWaves * 64) out[k] = sum[k];
 }
 
 // Fold the partial gradients in block order; with adam != 0 apply Adam.
 // grad_out (may be null) receives the folded gradient, loss_out the mean loss.
+// A workgroup folds 16 parameters: slice i of its 16 slices of 16 threads adds
+// every 16th partial, then the slices' sums are added in order.
 __global__ void __launch_bounds__(256)
 k_mlp_fold_adam(const float *__restrict__ partial, int nblocks, int64_t batch, int adam,
                 float *__restrict__ params, float *__restrict__ mom, float *__restrict__ vel,
                 float lr, float c1, float c2, float *__restrict__ grad_out,
                 double *__restrict__ loss_out) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ double part[16][17];
+    const int p = threadIdx.x & 15, slice = threadIdx.x >> 4;
+    const int k = blockIdx.x * 16 + p;
+    double acc = 0.0;  // the loss is summed in double; a double sum of floats costs nothing here
+    if (k <= kMlpParams) {
+#pragma unroll 4
+        for (int b = slice; b < nblocks; b += 16) acc += double(partial[size_t(b) * kGradLen + k]);
+    }
+    part[slice][p] = acc;
+    __syncthreads();
+    if (slice != 0 || k > kMlpParams) return;
+    double total = 0.0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) total += part[i][p];
     if (k == kMlpParams) {
-        double acc = 0.0;
-        for (int b = 0; b < nblocks; ++b) acc += double(partial[size_t(b) * kGradLen + kMlpParams]);
-        *loss_out = acc / double(batch);
+        *loss_out = total / double(batch);
         return;
     }
-    if (k > kMlpParams) return;
-    float g = 0.f;
-    for (int b = 0; b < nblocks; ++b) g += partial[size_t(b) * kGradLen + k];
+    const float g = float(total);
     if (grad_out) grad_out[k] = g;
     if (adam) {
         const float beta1 = 0.9f, beta2 = 0.999f, eps = 1e-8f;
@@ -214,12 +273,19 @@ int mfail(int code, const std::string &msg) {
 
 }  // namespace
 
+// Training workgroups of a batch: a unit per wavefront while CUs are free.
+static int grad_blocks(int64_t batch) {
+    const int64_t units = (batch + tlbm::kUnit - 1) / tlbm::kUnit;
+    const int64_t blocks = (units + tlbm::kGradWaves - 1) / tlbm::kGradWaves;
+    return int(blocks < tlbm::kGradBlocks ? blocks : tlbm::kGradBlocks);
+}
+
 struct tlbm_mlp_trainer {
     int64_t n = 0;
     float *X = nullptr, *T = nullptr, *params = nullptr, *mom = nullptr, *vel = nullptr;
     float *partial = nullptr, *grad = nullptr;
     double *loss = nullptr;
-    int max_blocks = 0;
+    int max_batch = 0, max_blocks = 0;
     int64_t steps = 0;
     uint64_t seed = 0;
     hipStream_t stream = nullptr;
@@ -236,7 +302,8 @@ int tlbm_mlp_trainer_create(const float *x, const float *t, int64_t n, const flo
     if (!tr) return mfail(TLBM_ENOMEM, "host allocation failed");
     tr->n = n;
     tr->seed = seed;
-    tr->max_blocks = (max_batch + tlbm::kTB - 1) / tlbm::kTB;
+    tr->max_batch = max_batch;
+    tr->max_blocks = grad_blocks((int64_t(max_batch) + 127) / 128 * 128);
     auto bail = [&](int rc) {
         tlbm_mlp_trainer_destroy(tr);
         return rc;
@@ -275,17 +342,19 @@ int tlbm_mlp_trainer_destroy(tlbm_mlp_trainer *tr) {
 
 int tlbm_mlp_trainer_step(tlbm_mlp_trainer *tr, int steps, int batch, float lr, double *last_loss) {
     if (!tr || steps < 0 || batch <= 0) return mfail(TLBM_EINVAL, "bad step arguments");
-    const int nb = (batch + tlbm::kTB - 1) / tlbm::kTB;
-    if (nb > tr->max_blocks) return mfail(TLBM_EINVAL, "batch larger than the trainer's max_batch");
+    // (whole units of 128 samples, as max_batch has always been rounded)
+    if ((int64_t(batch) + 127) / 128 > (int64_t(tr->max_batch) + 127) / 128)
+        return mfail(TLBM_EINVAL, "batch larger than the trainer's max_batch");
+    const int nb = grad_blocks(batch);
     for (int k = 0; k < steps; ++k) {
         ++tr->steps;
-        hipLaunchKernelGGL(tlbm::k_mlp_grad, dim3(nb), dim3(tlbm::kTB), 0, tr->stream, tr->X, tr->T,
+        hipLaunchKernelGGL(tlbm::k_mlp_grad, dim3(nb), dim3(tlbm::kGradWaves * 64), 0, tr->stream, tr->X, tr->T,
                            tr->n, int64_t(0), 1, tr->seed, tr->steps, int64_t(batch), tr->params,
                            tr->partial);
         MLP_HIP(hipGetLastError());
         const float c1 = 1.f - std::pow(0.9f, float(tr->steps));
         const float c2 = 1.f - std::pow(0.999f, float(tr->steps));
-        hipLaunchKernelGGL(tlbm::k_mlp_fold_adam, dim3((tlbm::kMlpParams + 1 + 255) / 256), dim3(256),
+        hipLaunchKernelGGL(tlbm::k_mlp_fold_adam, dim3((tlbm::kGradLen + 15) / 16), dim3(256),
                            0, tr->stream, tr->partial, nb, int64_t(batch), 1, tr->params, tr->mom,
                            tr->vel, lr, c1, c2, (float *)nullptr, tr->loss);
         MLP_HIP(hipGetLastError());
@@ -301,12 +370,13 @@ int tlbm_mlp_trainer_loss_grad(tlbm_mlp_trainer *tr, int64_t first, int64_t coun
                                float *grad) {
     if (!tr || first < 0 || count <= 0 || first + count > tr->n || !loss || !grad)
         return mfail(TLBM_EINVAL, "bad loss_grad arguments");
-    const int nb = int((count + tlbm::kTB - 1) / tlbm::kTB);
-    if (nb > tr->max_blocks) return mfail(TLBM_EINVAL, "count larger than the trainer's max_batch");
-    hipLaunchKernelGGL(tlbm::k_mlp_grad, dim3(nb), dim3(tlbm::kTB), 0, tr->stream, tr->X, tr->T, tr->n,
+    if ((count + 127) / 128 > (int64_t(tr->max_batch) + 127) / 128)
+        return mfail(TLBM_EINVAL, "count larger than the trainer's max_batch");
+    const int nb = grad_blocks(count);
+    hipLaunchKernelGGL(tlbm::k_mlp_grad, dim3(nb), dim3(tlbm::kGradWaves * 64), 0, tr->stream, tr->X, tr->T, tr->n,
                        first, 0, tr->seed, int64_t(0), count, tr->params, tr->partial);
     MLP_HIP(hipGetLastError());
-    hipLaunchKernelGGL(tlbm::k_mlp_fold_adam, dim3((tlbm::kMlpParams + 1 + 255) / 256), dim3(256), 0,
+    hipLaunchKernelGGL(tlbm::k_mlp_fold_adam, dim3((tlbm::kGradLen + 15) / 16), dim3(256), 0,
                        tr->stream, tr->partial, nb, count, 0, tr->params, tr->mom, tr->vel, 0.f, 1.f,
                        1.f, tr->grad, tr->loss);
     MLP_HIP(hipGetLastError());
