@@ -557,6 +557,50 @@ __device__ inline T edot(int ex, int ey, int ez, T ux, T uy, T uz) {
     return d;
 }
 
+// Products and sums are contracted only where fma_t says so.
+#define TLBM_ROUND_EACH _Pragma("clang fp contract(off)")
+
+// e_s.(c v) of FP32 values, C = c v rounded: a component after the first
+// enters with its product unrounded (e = (1, -1, *) of D3Q19 and D3Q27: the
+// first does, and the second rounded).
+template <class L, int S>
+__device__ inline float edot_scaled(float c, float vx, float vy, float vz, float Cx, float Cy, float Cz) {
+    TLBM_ROUND_EACH
+    constexpr int x = L::ex[S], y = L::ey[S], z = L::ez[S];
+    float t = 0.0f;
+    if constexpr (x != 0 && y != 0) {
+        if constexpr (L::Q != 15 && x > 0 && y < 0) t = fma_t(c, vx, -Cy);
+        else t = fma_t(y > 0 ? c : -c, vy, x > 0 ? Cx : -Cx);
+    } else if constexpr (x != 0) {
+        t = x > 0 ? Cx : -Cx;
+    } else if constexpr (y != 0) {
+        t = y > 0 ? Cy : -Cy;
+    }
+    if constexpr (z != 0)
+        t = (x != 0 || y != 0) ? fma_t(z > 0 ? c : -c, vz, t) : z > 0 ? Cz : -Cz;
+    return t;
+}
+
+// f_eq - w of FP32 storage, w (A + t + t^2 / (2 rho)) as in node_prepare, with
+// every rounding written out: all step kernels give a node the same bits, so
+// two steps in one pass and two passes agree, whatever the compiler makes of
+// either kernel.  t = e.(3 rho u) takes each product after the first into its
+// sum (D3Q19, D3Q27: for e = (1, -1, *) the first).
+template <class L>
+__device__ inline void equilibrium_f32(float (&feq)[L::Q], float dlt, float rho, float ux, float uy,
+                                       float uz, const float (&w)[L::Q]) {
+    TLBM_ROUND_EACH
+    const float usq = fma_t(uz, uz, fma_t(uy, uy, ux * ux));
+    const float A = fma_t(-(1.5f * rho), usq, dlt);
+    const float h = 0.5f * __builtin_amdgcn_rcpf(rho);
+    const float r3 = 3.0f * rho, Ux = r3 * ux, Uy = r3 * uy, Uz = r3 * uz;
+    each<0, L::Q>([&](auto s) {
+        TLBM_ROUND_EACH
+        const float t = s == 0 ? 0.0f : edot_scaled<L, s>(r3, ux, uy, uz, Ux, Uy, Uz);
+        feq[s] = w[s] * fma_t(t, fma_t(t, h, 1.0f), A);
+    });
+}
+
 // The reference's node update on registers, in phases.  f[] holds the
 // gathered pre-collision populations on entry (deviations d = f - w when
 // SHIFT).  node_prepare computes the moments and applies the node type's
@@ -647,8 +691,9 @@ __device__ inline bool node_prepare(T (&f)[L::Q], T (&feq)[L::Q], int t, T &rho,
             uz = num<T>(a.u_bc, a.fl.u_bc);
         }
         if constexpr (SHIFT) {
+            TLBM_ROUND_EACH
             dlt = inv_1mu * (c_in + (T(2) * s_in + sz));
-            rho = T(1) + dlt;
+            rho = fma_t(inv_1mu, c_in + (T(2) * s_in + sz), T(1));
         } else {
             rho = inv_1mu * (T(2) * s_in + sz);
         }
@@ -683,7 +728,9 @@ __device__ inline bool node_prepare(T (&f)[L::Q], T (&feq)[L::Q], int t, T &rho,
         });
     }
     // compute_equilibrium, LatticeStructure.hpp:92-103
-    {
+    if constexpr (SHIFT && !SC && sizeof(T) == 4) {
+        equilibrium_f32<L>(feq, dlt, rho, ux, uy, uz, w);
+    } else {
         const T usq = ux * ux + uy * uy + uz * uz;
         if constexpr (SHIFT) {
             // f_eq - w = w (delta + rho (cu + cu^2/2 - 3u^2/2)), cu = 3 e.u,
@@ -782,6 +829,13 @@ __device__ inline T smagorinsky_omega(const T (&pi)[6], const StepArgs &a) {
                         a.fl.nu;
         return __builtin_amdgcn_rcpf(3.f * (a.fl.nu + P * (1.f / 6.f)) + 0.5f);
     }
+    if constexpr (sizeof(T) == 4) {
+        TLBM_ROUND_EACH
+        const float n2 = fma_t(2.f, fma_t(pi[5], pi[5], fma_t(pi[3], pi[3], pi[4] * pi[4])),
+                               fma_t(pi[2], pi[2], fma_t(pi[1], pi[1], pi[0] * pi[0])));
+        const float P = sqrtf(fma_t(sqrtf(n2), a.fl.cs, a.fl.nu2)) - a.fl.nu;
+        return 1.f / fma_t(3.f, a.fl.nu + P / 6.f, 0.5f);
+    }
     T P = stress_norm<T>(pi);
     P *= num<T>(a.cs, a.fl.cs);
     P = sqrt(P + num<T>(a.nu2, a.fl.nu2)) - num<T>(a.nu, a.fl.nu);
@@ -797,7 +851,52 @@ __device__ inline void node_relax(T (&f)[L::Q], const T (&feq)[L::Q], T om) {
     });
 }
 
-// Whether a step kernel's fluid nodes relax conserving (fluid_pairs):
+// relax of a fluid node in FP32 storage, conserving to the rounding of
+// f - feq.  In exact arithmetic the mass and momentum of f - feq are small
+// values set by the weights (the reference's D3Q15/D3Q19 float weights do
+// not sum to 1); rounded FP32 equilibria miss them by a few ulp of feq, the
+// same amount at every node of a steady flow, and that residue accumulates
+// step after step (D3Q19 cylinder array: velocity L2 against FP64 1.6e-5
+// after 20000 steps).  The values are those of the weights w, not of their
+// float roundings: the D3Q27 weights sum to 1 in double but to 1 + 7.5e-9
+// in float, a mass source FP64 does not have.  The residue of mass m0 and
+// momentum m is taken out of f - feq as w_s (m0 + 3 e_s.m), which carries
+// that mass and momentum.
+template <class L>
+__device__ inline void node_relax_conserving(float (&f)[L::Q], const float (&feq)[L::Q],
+                                             const float (&w)[L::Q], float om, float rho,
+                                             float ux, float uy, float uz, const StepArgs &a) {
+    TLBM_ROUND_EACH
+    constexpr int Q = L::Q;
+    float nq[Q], m0 = -0.0f, mx = -0.0f, my = -0.0f, mz = -0.0f;
+    each<0, Q>([&](auto s) {
+        TLBM_ROUND_EACH
+        nq[s] = f[s] - feq[s];
+        m0 += nq[s];
+        if (L::ex[s] > 0) mx += nq[s]; else if (L::ex[s] < 0) mx -= nq[s];
+        if (L::ey[s] > 0) my += nq[s]; else if (L::ey[s] < 0) my -= nq[s];
+        if (L::ez[s] > 0) mz += nq[s]; else if (L::ez[s] < 0) mz -= nq[s];
+    });
+    const float usq = fma_t(uz, uz, fma_t(uy, uy, ux * ux));
+    m0 = fma_t(-rho, fma_t(1.5f * a.k1, usq, -a.k0), m0);
+    const float rk = rho * a.k2;
+    mx = fma_t(-rk, ux, mx);
+    my = fma_t(-rk, uy, my);
+    mz = fma_t(-rk, uz, mz);
+    const float Mx = 3.0f * mx, My = 3.0f * my, Mz = 3.0f * mz;
+    each<0, Q>([&](auto s) {
+        TLBM_ROUND_EACH
+        constexpr int x = L::ex[s], y = L::ey[s], z = L::ez[s];
+        float c = m0;
+        if constexpr (x * x + y * y + z * z == 1)
+            c = fma_t(3.0f * float(x + y + z), x ? mx : y ? my : mz, m0);
+        else if constexpr (s != 0)
+            c = m0 + edot_scaled<L, s>(3.0f, mx, my, mz, Mx, My, Mz);
+        f[s] = fma_t(-om, fma_t(-w[s], c, nq[s]), f[s]);
+    });
+}
+
+// Whether a step kernel's fluid nodes relax conserving:
 // FP32 storage.  FP16's own rounding is stochastic, no bias; its float
 // weights get the mass and momentum balance of w from the equilibrium
 // corrections dt3, dk0, dk1 instead, at a fraction of the cost (the
@@ -812,8 +911,6 @@ __device__ inline float rcp_newton(float x) {
     const float r = __builtin_amdgcn_rcpf(x);
     return fma_t(r, fma_t(-x, r, 1.0f), r);
 }
-
-#define TLBM_ROUND_EACH _Pragma("clang fp contract(off)")
 
 // ---- deviation storage: the node update by direction pairs ---------------------------------
 // A direction s and its opposite b = bb[s] have the same weight w and the
@@ -1071,15 +1168,26 @@ __device__ inline void pairs_relax(T (&f)[L::Q], const T (&n)[L::Q], uint64_t so
     }
 }
 
+// Deviation storages update their nodes by direction pairs, except FP32 D3Q15
+// and D3Q19 without the network, which go direction by direction
+// (equilibrium_f32, node_relax_conserving).  Both forms are as accurate, but
+// tau near 1/2 grows the difference of two roundings by orders of magnitude in
+// a few hundred steps, so a form is kept where it costs little: D3Q19
+// 128x128x512 154 against 145 us per step by pairs (165 against 149 with
+// Smagorinsky), D3Q15 125 against 118.  D3Q27 goes by pairs: 207 against 254 us
+// (192^3, Smagorinsky), whose registers leave no room for the other form.
+template <int ST, int Q>
+constexpr bool kPairForm = !(ST == ST_F32 && Q != 27);
+
 // The whole reference update of one node (TLBM_Partition.cpp:742-807).
-// CONSERVE: fluid nodes relax with node_relax_conserving.  SC: the scaled
-// form of node_prepare (the relaxation is the same in either scale).
-template <class L, class T, bool SHIFT, bool COLLIDE, bool CONSERVE = false, bool SC = false>
+// CONSERVE: fluid nodes relax conserving.  SC: the scaled form of node_prepare
+// (the relaxation is the same in either scale).  PAIRS: by direction pairs.
+template <class L, class T, bool SHIFT, bool COLLIDE, bool CONSERVE = false, bool SC = false, bool PAIRS = true>
 __device__ inline void node_update(T (&f)[L::Q], int t, T &rho, T &ux, T &uy, T &uz,
                                    const StepArgs &a, const T *__restrict__ uy_head,
                                    const T (&w)[L::Q], uint32_t g) {
     static_assert(!(SC && CONSERVE), "the conserving relax works on d");
-    if constexpr (COLLIDE && SHIFT) {
+    if constexpr (COLLIDE && SHIFT && PAIRS) {
         T n[L::Q], om = num<T>(a.omega, a.fl.omega);
         const uint64_t solids = __ballot(t == 1);
         pairs_prepare<L, T, SC, CONSERVE>(f, n, t, a, uy_head, w, g);
@@ -1100,7 +1208,15 @@ __device__ inline void node_update(T (&f)[L::Q], int t, T &rho, T &ux, T &uy, T 
         node_stress<L, T, SC>(f, feq, pi, w);
         om = smagorinsky_omega<T, SC>(pi, a);
     }
-    if (a.dynamics == 1) node_relax<L, T>(f, feq, om);
+    if (a.dynamics == 1) {
+        if constexpr (CONSERVE) {
+            if (t == 0) {
+                node_relax_conserving<L>(f, feq, w, om, rho, ux, uy, uz, a);
+                return;
+            }
+        }
+        node_relax<L, T>(f, feq, om);
+    }
 }
 
 // Has the step kernels' prologue load, in one batch of scalar loads, the
@@ -1183,8 +1299,8 @@ k_lbm(const typename StorageT<ST>::st *__restrict__ fin, typename StorageT<ST>::
     const int t = type_final<MODE>(t0, nd_type, chunk_type, g);
     T rho, ux, uy, uz;
     if (MODE == MODE_STEP) {
-        node_update<L, T, S::kShift, true, kConserve<ST, Q>, S::kScaled>(f, t, rho, ux, uy, uz, a,
-                                                                         uy_head, w, g);
+        node_update<L, T, S::kShift, true, kConserve<ST, Q>, S::kScaled, kPairForm<ST, Q>>(
+            f, t, rho, ux, uy, uz, a, uy_head, w, g);
         const PushOut<L, ST> po(fout, (blk * BS) >> StorageT<ST>::kCB, g);
         const uint32_t rs = ST == ST_F16 ? round_stream(g, a.step) : 0u;
         each<0, Q>([&](auto s) { po.template store<NTSTORE>(s, S::step_out(f[s], s, a, rs + uint32_t(s) * kStreamStep)); });
