@@ -11,6 +11,7 @@
 #include <string>
 #include <vector>
 
+#include "host_copy.h"
 #include "launch.h"
 #include "pair_plan.h"
 
@@ -155,6 +156,7 @@ struct tlbm_gpu {
     double *partial = nullptr;  // reduction partials
     int nparts = 0;
     bool has_lid = false;
+    bool copies = false;  // holds a share of the host copy rings
     long long steps_since_set = 0;
     uint64_t step_count = 0;  // steps since creation (FP16 rounding stream)
     hipStream_t stream = nullptr;
@@ -374,6 +376,8 @@ int tlbm_gpu_create(const tlbm_params *p, const uint8_t *nd_type, tlbm_gpu **out
         return cleanup_fail(fail(TLBM_EHIP, std::string("init sync: ") + hipGetErrorString(e)));
     h->cur = 0;
     h->steps_since_set = 0;
+    tlbm::host_copy_retain();
+    h->copies = true;
     *out = h;
     return TLBM_OK;
 }
@@ -396,6 +400,7 @@ int tlbm_gpu_destroy(tlbm_gpu *h) {
     if (h->ev0) (void)hipEventDestroy(h->ev0);
     if (h->ev1) (void)hipEventDestroy(h->ev1);
     if (h->stream) (void)hipStreamDestroy(h->stream);
+    if (h->copies) tlbm::host_copy_release();
     delete h;
     return TLBM_OK;
 }
@@ -467,22 +472,16 @@ int tlbm_gpu_sync(tlbm_gpu *h) {
     return TLBM_OK;
 }
 
-// Copy `count` compute-type values from device `src` into host doubles.
-static int download_as_double(tlbm_gpu *h, const void *src, size_t count, double *const *dst,
-                              int nplanes) {
-    const size_t esz = size_t(h->ops->macro_bytes);
-    std::vector<unsigned char> tmp(esz * count * nplanes);
-    TLBM_HIP(hipMemcpyAsync(tmp.data(), src, tmp.size(), hipMemcpyDeviceToHost, h->stream));
-    TLBM_HIP(hipStreamSynchronize(h->stream));
-    for (int k = 0; k < nplanes; ++k) {
-        if (!dst[k]) continue;
-        if (esz == 8) {
-            std::memcpy(dst[k], tmp.data() + size_t(k) * count * 8, count * 8);
-        } else {
-            const float *fp = reinterpret_cast<const float *>(tmp.data()) + size_t(k) * count;
-            for (size_t i = 0; i < count; ++i) dst[k][i] = double(fp[i]);
-        }
-    }
+// nplanes (at most 4) planes of `count` values at `src` (compute type if
+// `compute`, else doubles) into the caller's arrays; null ones are left out.
+static int download_planes(tlbm_gpu *h, const void *src, size_t count, bool compute, double *const *dst,
+                           int nplanes) {
+    const size_t esz = compute ? size_t(h->ops->macro_bytes) : sizeof(double);
+    tlbm::CopyPart parts[4];
+    int n = 0;
+    for (int k = 0; k < nplanes; ++k)
+        if (dst[k]) parts[n++] = {static_cast<const char *>(src) + size_t(k) * count * esz, dst[k], count};
+    TLBM_HIP(tlbm::copy_to_host(parts, n, esz == 4, h->stream));
     return TLBM_OK;
 }
 
@@ -500,7 +499,7 @@ int tlbm_gpu_get_macros(tlbm_gpu *h, double *ux, double *uy, double *uz, double 
                                h->macro, nullptr, h->args, h->stream);
     if (e != hipSuccess) return fail(TLBM_EHIP, std::string("moments: ") + hipGetErrorString(e));
     double *dst[4] = {ux, uy, uz, rho};
-    return download_as_double(h, h->macro, h->N, dst, 4);
+    return download_planes(h, h->macro, h->N, true, dst, 4);
 }
 
 int tlbm_gpu_get_forces(tlbm_gpu *h, double *fx, double *fy, double *fz) {
@@ -510,11 +509,7 @@ int tlbm_gpu_get_forces(tlbm_gpu *h, double *fx, double *fy, double *fz) {
     hipError_t e = h->ops->forces(h->Q, h->f[h->cur], h->nd, h->staging, h->args, h->stream);
     if (e != hipSuccess) return fail(TLBM_EHIP, std::string("forces: ") + hipGetErrorString(e));
     double *dst[3] = {fx, fy, fz};
-    for (int k = 0; k < 3; ++k)
-        TLBM_HIP(hipMemcpyAsync(dst[k], h->staging + size_t(k) * h->N, size_t(h->N) * 8,
-                                hipMemcpyDeviceToHost, h->stream));
-    TLBM_HIP(hipStreamSynchronize(h->stream));
-    return TLBM_OK;
+    return download_planes(h, h->staging, h->N, false, dst, 3);
 }
 
 int tlbm_gpu_get_populations(tlbm_gpu *h, double *f) {
@@ -524,9 +519,7 @@ int tlbm_gpu_get_populations(tlbm_gpu *h, double *f) {
     if (int rc = ensure_staging(h, b)) return rc;
     hipError_t e = h->ops->get_populations(h->Q, h->f[h->cur], h->staging, h->args, h->stream);
     if (e != hipSuccess) return fail(TLBM_EHIP, std::string("get populations: ") + hipGetErrorString(e));
-    TLBM_HIP(hipMemcpyAsync(f, h->staging, b, hipMemcpyDeviceToHost, h->stream));
-    TLBM_HIP(hipStreamSynchronize(h->stream));
-    return TLBM_OK;
+    return download_planes(h, h->staging, size_t(h->N) * h->Q, false, &f, 1);
 }
 
 int tlbm_gpu_set_populations(tlbm_gpu *h, const double *f) {
@@ -625,11 +618,7 @@ int tlbm_gpu_get_time_average(tlbm_gpu *h, double *u, double *v, double *w, doub
     if (int rc = check(h)) return rc;
     if (!h->avg) return fail(TLBM_ESTATE, "time averaging was never enabled");
     double *dst[4] = {u, v, w, rho};
-    for (int k = 0; k < 4; ++k)
-        if (dst[k])
-            TLBM_HIP(hipMemcpyAsync(dst[k], h->avg + size_t(k) * h->N, size_t(h->N) * sizeof(double),
-                                    hipMemcpyDeviceToHost, h->stream));
-    TLBM_HIP(hipStreamSynchronize(h->stream));
+    if (int rc = download_planes(h, h->avg, h->N, false, dst, 4)) return rc;
     if (nsteps) *nsteps = h->avg_steps;
     return TLBM_OK;
 }
@@ -710,9 +699,7 @@ int tlbm_gpu_box_filter(tlbm_gpu *h, double *out) {
     if (int rc = ensure_staging(h, ob)) return rc;
     e = h->ops->box_filter(h->filt_in, h->staging, h->args, h->stream);
     if (e != hipSuccess) return fail(TLBM_EHIP, std::string("box filter: ") + hipGetErrorString(e));
-    TLBM_HIP(hipMemcpyAsync(out, h->staging, ob, hipMemcpyDeviceToHost, h->stream));
-    TLBM_HIP(hipStreamSynchronize(h->stream));
-    return TLBM_OK;
+    return download_planes(h, h->staging, ob / sizeof(double), false, &out, 1);
 }
 
 int tlbm_gpu_memory_bytes(const tlbm_gpu *h, uint64_t *bytes) {
