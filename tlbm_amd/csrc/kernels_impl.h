@@ -42,6 +42,11 @@ struct Launch {
                                    nd, chunk_type, mac, uyh, a);
             }
             break;
+        case MODE_STEP_AVG:
+            if (a.closure) return hipErrorInvalidValue;
+            hipLaunchKernelGGL((k_lbm<L, ST, MODE_STEP_AVG, false, TU::kNTLoad>), dim3(blocks_for(a.N)),
+                               dim3(kBlock), 0, s, in, out, nd, chunk_type, mac, uyh, a);
+            break;
         case MODE_MACROS:
             hipLaunchKernelGGL((k_lbm<L, ST, MODE_MACROS>), dim3(blocks_for(a.N)), dim3(kBlock), 0,
                                s, in, out, nd, nullptr, mac, uyh, a);

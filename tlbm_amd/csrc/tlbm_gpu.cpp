@@ -431,12 +431,15 @@ static int queue_steps(tlbm_gpu *h, int nsteps) {
             if (e != hipSuccess) return fail(TLBM_EHIP, std::string("type-5 helper: ") + hipGetErrorString(e));
         }
         h->args.step = uint32_t(h->step_count++);
-        hipError_t e = h->ops->lbm(h->Q, tlbm::MODE_STEP, fin, fout, h->nd, h->chunk_type, nullptr,
-                                   h->uy_head, h->args, h->stream);
+        // the time average's sums in the same pass; with the network, after it
+        const bool fused = h->avg_on && !net;
+        hipError_t e = h->ops->lbm(h->Q, fused ? tlbm::MODE_STEP_AVG : tlbm::MODE_STEP, fin, fout, h->nd,
+                                   h->chunk_type, fused ? h->avg : nullptr, h->uy_head, h->args, h->stream);
         if (e != hipSuccess) return fail(TLBM_EHIP, std::string("stream-collide: ") + hipGetErrorString(e));
         h->cur = 1 - h->cur;
         ++h->steps_since_set;
-        if (h->avg_on) {
+        if (fused) ++h->avg_steps;
+        if (h->avg_on && !fused) {
             // the step just read f[1-cur]; its moments go into the sums
             e = h->ops->lbm(h->Q, tlbm::MODE_AVG, h->f[1 - h->cur], nullptr, h->nd, nullptr, h->avg,
                             nullptr, h->args, h->stream);
