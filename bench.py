@@ -7,8 +7,9 @@ radius 12, centred at (y, z) = (64, 128), bounce-back cylinder, Zou-He
 velocity inlet u_z = 0.04 at z = 0, pressure outlet rho = 1 at z = 511,
 tau = 0.55, starting from rest (f = w).
 
-A step is one fused stream-collide launch over the whole lattice with the
-populations resident in HBM.  The headline `value` is MLUPS with FP32
+A step is one fused stream-collide update of the whole lattice with the
+populations resident in HBM; FP32, FP64 and FP32X take two steps per launch
+(all but a call's last one or two), FP16 one.  The headline `value` is MLUPS with FP32
 storage (nx*ny*nz*steps / wall time of the timed steps); FP64, FP16 (f - w)
 and FP32X storage run the same timed steps, reported under `variants`.
 After the timed region every storage runs the configuration's full 20000
@@ -16,9 +17,10 @@ steps from rest on the full lattice (--accuracy-steps), and each reduced
 storage reports its velocity L2 over fluid nodes, its mass drift (FP64
 on-device sums) and the reference's own validation metric, the relative
 1-norm difference of the speed |u| over all nodes (python/validate.py:33-43),
-against the FP64 run.  `roofline` prices the FP32 kernel at 2*Q*4 = 152
-algorithmic bytes per lattice update against 8 TB/s, with its average
-duration from HIP events on the stream the kernel runs on.
+against the FP64 run.  `roofline` prices the FP32 kernel at the 2*Q*4 = 152
+bytes that each node's populations take to read and write once per launch,
+i.e. 76 per lattice update, against 8 TB/s, with the average duration of a
+step from HIP events on the stream the kernel runs on.
 `cpu_baseline` times the reference's own MPI executable (built from its
 sources into oracle/_ref) on the host's physical cores (those this process
 may run on, at most its CPU share) for 200 steps of the same lattice, or the
@@ -45,6 +47,8 @@ from tlbm_amd.gpu import BYTES_PER_VALUE, Lattice  # noqa: E402
 
 METRIC = "D3Q19 MLUPS & %HBM roofline, FP32/FP16 vs FP64 at stated L2 error"
 PEAK_HBM_GBS = 8000.0
+# steps of the timed lattice that one launch takes
+STEPS_PER_LAUNCH = {"f64": 2, "f32": 2, "f32x": 2, "f16": 1}
 Q = 19
 NX, NY, NZ = 128, 128, 512
 TAU = 0.55
@@ -275,13 +279,17 @@ def main():
     head = storages[0]
     h = res[head]
     n = NX * NY * NZ
-    b_alg = 2 * Q * BYTES_PER_VALUE[head]
+    def bytes_per_update(st):
+        return 2 * Q * BYTES_PER_VALUE[st] // STEPS_PER_LAUNCH[st]
+
+    b_alg = bytes_per_update(head)
     achieved = b_alg * n / (h["kernel_ms"] * 1e-3) / 1e9
     variants = {}
     for st, r in res.items():
         variants[st] = {"mlups": round(r["mlups"], 1), "kernel_ms": round(r["kernel_ms"], 5),
-                        "bytes_per_update": 2 * Q * BYTES_PER_VALUE[st],
-                        "hbm_frac": round(2 * Q * BYTES_PER_VALUE[st] * n / (r["kernel_ms"] * 1e-3)
+                        "bytes_per_update": bytes_per_update(st),
+                        "steps_per_launch": STEPS_PER_LAUNCH[st],
+                        "hbm_frac": round(bytes_per_update(st) * n / (r["kernel_ms"] * 1e-3)
                                           / 1e9 / PEAK_HBM_GBS, 4)}
     if args.accuracy_steps > 0:
         for st, e in accuracy_runs(nd, storages, args.accuracy_steps).items():
