@@ -37,6 +37,15 @@ struct Launch {
                                        out, nd, chunk_type, uyh, a);
                 }
             } else {
+                if constexpr (TU::kSmallN > 0) {
+                    if (a.N < TU::kSmallN) {
+                        constexpr int SBS = TU::kSmallBS;
+                        hipLaunchKernelGGL((k_lbm<L, ST, MODE_STEP_SMALL, false, TU::kNTLoad, true, SBS>),
+                                           dim3((a.N + SBS - 1) / SBS), dim3(SBS), 0, s, in, out, nd,
+                                           chunk_type, mac, uyh, a);
+                        break;
+                    }
+                }
                 hipLaunchKernelGGL((k_lbm<L, ST, MODE_STEP, false, TU::kNTLoad, true, TU::kBS>),
                                    dim3((a.N + TU::kBS - 1) / TU::kBS), dim3(TU::kBS), 0, s, in, out,
                                    nd, chunk_type, mac, uyh, a);

@@ -44,7 +44,8 @@
 namespace tlbm {
 
 enum Storage : int { ST_F64 = 0, ST_F32 = 1, ST_F16 = 2, ST_F32X = 3 };
-enum Mode : int { MODE_STEP = 0, MODE_MACROS = 1, MODE_HEAD = 2, MODE_AVG = 3, MODE_STRESS = 4, MODE_STEP_AVG = 5 };
+enum Mode : int { MODE_STEP = 0, MODE_MACROS = 1, MODE_HEAD = 2, MODE_AVG = 3, MODE_STRESS = 4, MODE_STEP_AVG = 5,
+                  MODE_STEP_SMALL = 6 };
 
 constexpr int kBlock = 256;  // 4 wave64 per workgroup
 constexpr int kRed = 7;      // values per FP64 reduction partial
@@ -320,22 +321,38 @@ constexpr uint32_t kStreamStep = 0x9E3779B9u;
 // non-temporal loads (D3Q27 145.0 against 153.8); FP32 D3Q19 202.9 against 205.0, D3Q27 2.05 against
 // 2.17 ms.  Every kernel stores
 // non-temporally.
+// Lattices of less than kSmallN nodes take workgroups of kSmallBS threads.
+// FP64: 256 threads spread a small lattice over more CUs and let a CU start
+// the next workgroup sooner.  us per step with 1024 threads (D3Q27 512) and
+// with 256: D3Q15 24x24x96 7.3 and 6.0, 48x48x64 9.55 and 7.6, 96^3 39.5 and
+// 38.3; D3Q19 24x24x96 9.25 and 6.3, 64x64x96 23.5 and 21.6, 95x83x120 53.3
+// and 52.9; D3Q27 48x48x64 18.4 and 12.5, 96^3 71.8 and 68.2.  Beyond 2^20
+// nodes the large ones are ahead (above).  64 threads are 0.1 us faster on the
+// smallest lattices and 2 to 7 % slower from 80^3 on.
 template <int ST, int Q> struct Tune;
 template <int Q> struct Tune<ST_F64, Q> {
     static constexpr int kBS = Q == 27 ? 512 : 1024;
     static constexpr bool kNTLoad = Q != 27;
+    static constexpr int kSmallBS = 256;
+    static constexpr uint32_t kSmallN = 1u << 20;
 };
 template <int Q> struct Tune<ST_F32, Q> {
     static constexpr int kBS = 256;
     static constexpr bool kNTLoad = false;
+    static constexpr int kSmallBS = kBS;
+    static constexpr uint32_t kSmallN = 0;
 };
 template <int Q> struct Tune<ST_F32X, Q> {
     static constexpr int kBS = 256;
     static constexpr bool kNTLoad = false;
+    static constexpr int kSmallBS = kBS;
+    static constexpr uint32_t kSmallN = 0;
 };
 template <int Q> struct Tune<ST_F16, Q> {
     static constexpr int kBS = 256;
     static constexpr bool kNTLoad = false;
+    static constexpr int kSmallBS = kBS;
+    static constexpr uint32_t kSmallN = 0;
 };
 
 // Workgroup -> node block.  The dispatcher deals workgroups round-robin to
@@ -1237,7 +1254,8 @@ __device__ inline void load_args_early(const StepArgs &a, const void *fin) {
 // fin -> fout; MODE_MACROS recomputes the moments of the step that read fin
 // (ux, uy, uz, rho planes of N compute-type values in `out`); MODE_AVG adds
 // those moments to four planes of N doubles in `out` (time average);
-// MODE_STEP_AVG does both in one pass: the sums' planes are read behind the
+// MODE_STEP_SMALL is MODE_STEP for lattices below Tune::kSmallN (a kernel of
+// its own in traces and register listings); MODE_STEP_AVG does both in one pass: the sums' planes are read behind the
 // gathers, and the state is not gathered a second time (D3Q19 FP32
 // 95x83x241 90 -> 69 us per averaged step, FP64 174 -> 115, FP16 128x128x256
 // 120 -> 90, FP64 D3Q15 64x64x96 34 -> 21);
@@ -1252,8 +1270,9 @@ __device__ inline void load_args_early(const StepArgs &a, const void *fin) {
 template <class L, int ST, int MODE, bool REMAP = true, bool NTLOAD = false, bool NTSTORE = true,
           int BS = kBlock>
 __global__ void __launch_bounds__(BS)
-__attribute__((amdgpu_waves_per_eu(MODE == MODE_STEP ? kStepWaves<ST, L::Q> : 1,
-                                   MODE == MODE_STEP ? kStepWavesMax<ST, L::Q> : 8)))
+__attribute__((amdgpu_waves_per_eu(
+    MODE == MODE_STEP || MODE == MODE_STEP_SMALL ? kStepWaves<ST, L::Q> : 1,
+    MODE == MODE_STEP || MODE == MODE_STEP_SMALL ? kStepWavesMax<ST, L::Q> : 8)))
 k_lbm(const typename StorageT<ST>::st *__restrict__ fin, typename StorageT<ST>::st *__restrict__ fout,
       const uint8_t *__restrict__ nd_type, const uint8_t *__restrict__ chunk_type,
       void *__restrict__ out, const typename StorageT<ST>::T *__restrict__ uy_head, StepArgs a) {
@@ -1261,7 +1280,7 @@ k_lbm(const typename StorageT<ST>::st *__restrict__ fin, typename StorageT<ST>::
     using T = typename S::T;
     using st = typename S::st;
     constexpr int Q = L::Q;
-    constexpr bool kStep = MODE == MODE_STEP || MODE == MODE_STEP_AVG;
+    constexpr bool kStep = MODE == MODE_STEP || MODE == MODE_STEP_SMALL || MODE == MODE_STEP_AVG;
     constexpr int kType = kStep ? MODE_STEP : MODE;  // how the node type is read
     if (kStep) load_args_early(a, fin);
     if constexpr (kStep && kGatherPrio<ST, Q>) __builtin_amdgcn_s_setprio(3);
