@@ -198,3 +198,18 @@ def test_step_raises_wave_priority_where_measured(code, lattice, storage, raised
     """s_setprio 3 while the gathers go out, exactly where it measured faster."""
     ins = _step(code, lattice, storage)
     assert ("s_setprio 3" in ins) == raised
+
+
+def _pair(code):
+    """The two-step pass's kernels."""
+    found = {k: v for k, v in code.items() if k.startswith("_ZN4tlbm10k_lbm_pair")}
+    assert found
+    return found
+
+
+def test_two_step_pass_has_no_lid_rule(code):
+    """A lattice with a type-5 node never takes the two-step pass, whose
+    uy_head is null: the rule's reads through it (flat loads; all others are
+    global, buffer or LDS accesses) are not in the kernels."""
+    for name, ins in _pair(code).items():
+        assert not [x for x in ins if x.startswith("flat_load")], name

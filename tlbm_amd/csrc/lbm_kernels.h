@@ -732,7 +732,7 @@ __device__ inline bool node_prepare(T (&f)[L::Q], T (&feq)[L::Q], int t, T &rho,
         }
     }
     if (!COLLIDE) return true;
-    if (t == 5) {
+    if (uy_head && t == 5) {  // no lattice with this type takes the two-step pass, which has no uy_head
         // set_uz_bc (LatticeStructure.hpp:166-177); the y term reads uy of
         // node s of this step, as the reference's uy[spd] does
         const T ubc = a.inlet_uz ? T(a.inlet_uz[g % a.nxny]) : num<T>(a.u_bc, a.fl.u_bc);
