@@ -7,12 +7,8 @@ tiles that overhang the lattice in x and y, z segments of unequal length, the
 periodic wrap in x, y and z across tiles, walls, an obstacle across a tile's
 edge, inlet (with and without a profile) and outlet, and both tile widths.
 
-Both run the same node update on the same values: FP64 agrees bitwise.  The
-other storages are compiled for both kernels apart, and the compiler may
-contract a product into one and not into the other: one rounding (2^-24) of a
-population per step, a few per population after 7 steps.  With the network
-such a rounding may move a bf16 rounding of a hidden unit (2^-9 of it), of
-which the relaxation rate passes on a small part."""
+Both run the same node update on the same values, with every rounding written
+out, so they agree bit for bit in every storage, with the network too."""
 import numpy as np
 import pytest
 
@@ -62,14 +58,6 @@ def test_two_step_pass_matches_single_steps(gpu_lib, q, storage, dims, cs, netwo
             red = lat.reduce()
             out.append((lat.populations(), lat.macros(), red["residual"], red["mass"]))
     (fa, ma, ra, sa), (fb, mb, rb, sb) = out
-    if storage == "f64":
-        assert np.array_equal(fa, fb)
-        assert all(np.array_equal(ma[k], mb[k]) for k in ma)
-        assert ra == rb
-        return
-    # f0 is of order w <= 1/3; 7 steps, each a handful of roundings of at most
-    # 2^-24 of that (the stored d = f - w is smaller still)
-    tol = 3e-4 if network else 7 * 8 * 2.0 ** -24 / 3
-    assert np.max(np.abs(fa - fb)) <= tol
-    assert max(np.max(np.abs(ma[k] - mb[k])) for k in ma) <= q * tol
-    assert abs(ra / rb - 1.0) <= 1e-4 and abs(sa / sb - 1.0) <= 1e-7
+    assert np.array_equal(fa, fb)
+    assert all(np.array_equal(ma[k], mb[k]) for k in ma)
+    assert ra == rb and sa == sb

@@ -67,12 +67,8 @@ template <int ST> constexpr bool kClosureNTLoad = (ST == ST_F16);
 // (6).  FP32 D3Q27 stays at 4: at 5 it spills (325 against 299 us).
 template <int ST, int Q>
 constexpr int kClosureWaves = Q == 27 ? (ST == ST_F16 ? 5 : 4) : (ST == ST_F32 && Q == 19 ? 5 : 6);
-// Waves per SIMD the step is register-allocated for (least and most).  FP16
-// left alone takes 96 VGPRs for D3Q19 (114 against 102 us per step); FP32
-// D3Q19, HBM-bound, loses with more than 5 (68 VGPRs, 7 waves: 206.7 against
-// 202.6 us).
-template <int ST, int Q>
-constexpr int kStepWaves = ST == ST_F16 ? (Q == 27 ? 6 : 8) : ST == ST_F32 && Q == 15 ? 8 : 1;
+// Most waves per SIMD the step is register-allocated for: FP32 D3Q19,
+// HBM-bound, loses with more than 5 (7 waves 206.7 against 202.6 us per step).
 template <int ST, int Q>
 constexpr int kStepWavesMax = ST == ST_F32 && Q == 19 ? 5 : 8;
 // Steps with kTypeAhead, and the closure collide in every storage, load the
@@ -552,14 +548,6 @@ template <int A, int B, class F>
 __device__ inline void each(F &&f) {
     each_impl<A>(f, std::make_integer_sequence<int, B - A>{});
 }
-// ... for the first direction of every pair of opposite directions.
-template <class L, class F>
-__device__ inline void each_pair(F &&f) {
-    each<1, L::Q>([&](auto k) {
-        if constexpr (k < L::bb[k]) f(k);
-    });
-}
-
 // a * b + c rounded once.
 __device__ inline float fma_t(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ inline double fma_t(double a, double b, double c) { return __builtin_fma(a, b, c); }
@@ -577,44 +565,68 @@ __device__ inline T edot(int ex, int ey, int ez, T ux, T uy, T uz) {
 // Products and sums are contracted only where fma_t says so.
 #define TLBM_ROUND_EACH _Pragma("clang fp contract(off)")
 
-// e_s.(c v) of FP32 values, C = c v rounded: a component after the first
-// enters with its product unrounded (e = (1, -1, *) of D3Q19 and D3Q27: the
-// first does, and the second rounded).
-template <class L, int S>
-__device__ inline float edot_scaled(float c, float vx, float vy, float vz, float Cx, float Cy, float Cz) {
-    TLBM_ROUND_EACH
-    constexpr int x = L::ex[S], y = L::ey[S], z = L::ez[S];
-    float t = 0.0f;
-    if constexpr (x != 0 && y != 0) {
-        if constexpr (L::Q != 15 && x > 0 && y < 0) t = fma_t(c, vx, -Cy);
-        else t = fma_t(y > 0 ? c : -c, vy, x > 0 ? Cx : -Cx);
-    } else if constexpr (x != 0) {
-        t = x > 0 ? Cx : -Cx;
-    } else if constexpr (y != 0) {
-        t = y > 0 ? Cy : -Cy;
-    }
-    if constexpr (z != 0)
-        t = (x != 0 || y != 0) ? fma_t(z > 0 ? c : -c, vz, t) : z > 0 ? Cz : -Cz;
-    return t;
+// Whether e_s.(c v) rounds the product of y, not that of x, by itself.
+template <class L, bool STEP>
+constexpr bool rounds_y(int s) {
+    return L::Q != 15 && L::ex[s] > 0 && L::ey[s] != 0 && (!STEP || L::ey[s] < 0);
 }
 
-// f_eq - w of FP32 storage, w (A + t + t^2 / (2 rho)) as in node_prepare, with
-// every rounding written out: all step kernels give a node the same bits, so
-// two steps in one pass and two passes agree, whatever the compiler makes of
-// either kernel.  t = e.(3 rho u) takes each product after the first into its
-// sum (D3Q19, D3Q27: for e = (1, -1, *) the first).
-template <class L>
-__device__ inline void equilibrium_f32(float (&feq)[L::Q], float dlt, float rho, float ux, float uy,
-                                       float uz, const float (&w)[L::Q]) {
+// e_s.(c v), C = c v rounded: of a sum's products the first is rounded, the
+// others enter unrounded (rounds_y: of x and y the second is rounded).
+// Opposite directions that round alike share one value.
+template <class L, int S, bool STEP, class T>
+__device__ inline T edot_scaled(T c, T vx, T vy, T vz, T Cx, T Cy, T Cz) {
     TLBM_ROUND_EACH
-    const float usq = fma_t(uz, uz, fma_t(uy, uy, ux * ux));
-    const float A = fma_t(-(1.5f * rho), usq, dlt);
-    const float h = 0.5f * __builtin_amdgcn_rcpf(rho);
-    const float r3 = 3.0f * rho, Ux = r3 * ux, Uy = r3 * uy, Uz = r3 * uz;
+    constexpr int x = L::ex[S], y = L::ey[S], z = L::ez[S];
+    if constexpr (L::bb[S] < S && rounds_y<L, STEP>(S) == rounds_y<L, STEP>(L::bb[S])) {
+        return -edot_scaled<L, L::bb[S], STEP>(c, vx, vy, vz, Cx, Cy, Cz);
+    } else {
+        T t = T(0);
+        if constexpr (x != 0 && y != 0) {
+            if constexpr (rounds_y<L, STEP>(S)) t = fma_t(c, vx, y > 0 ? Cy : -Cy);
+            else t = fma_t(y > 0 ? c : -c, vy, x > 0 ? Cx : -Cx);
+        } else if constexpr (x != 0) {
+            t = x > 0 ? Cx : -Cx;
+        } else if constexpr (y != 0) {
+            t = y > 0 ? Cy : -Cy;
+        }
+        if constexpr (z != 0)
+            t = (x != 0 || y != 0) ? fma_t(z > 0 ? c : -c, vz, t) : z > 0 ? Cz : -Cz;
+        return t;
+    }
+}
+
+// u^2 (STEP: with u_x^2 rounded by itself, else u_y^2).
+template <bool STEP, class T>
+__device__ inline T speed2(T ux, T uy, T uz) {
+    TLBM_ROUND_EACH
+    return fma_t(uz, uz, STEP ? fma_t(uy, uy, ux * ux) : fma_t(ux, ux, uy * uy));
+}
+
+// f_eq - w of FP32 and FP32X storage, w (A + t + t^2 / (2 rho)) as in
+// node_prepare.  Here and in all that the deviation storages compute, every
+// rounding is written out: a node's bits are the same in each kernel, so that
+// two steps in one pass and two passes agree, whatever the compiler makes of
+// either.  Which product of a sum is rounded by itself is no matter of
+// accuracy.  It is as in the package's first version, and there the step
+// (STEP) differs from the network's step and the stress planes (not STEP): a
+// flow near tau = 1/2 grows a last-bit difference by orders of magnitude in a
+// few hundred steps, FP16's stochastic rounding and the network's bf16 units
+// flip on one, and a run could not be compared with an earlier one.
+template <class L, bool STEP, class T>
+__device__ inline void equilibrium_dev(T (&feq)[L::Q], T dlt, T rho, T ux, T uy, T uz, const T (&w)[L::Q]) {
+    TLBM_ROUND_EACH
+    const T A = fma_t(-(T(1.5) * rho), speed2<STEP>(ux, uy, uz), dlt);
+    T h;
+    if constexpr (sizeof(T) == 8)
+        h = T(0.5) / rho;  // FP32X: every operation in FP64
+    else
+        h = T(0.5) * __builtin_amdgcn_rcpf(rho);
+    const T r3 = T(3) * rho, Ux = r3 * ux, Uy = r3 * uy, Uz = r3 * uz;
     each<0, L::Q>([&](auto s) {
         TLBM_ROUND_EACH
-        const float t = s == 0 ? 0.0f : edot_scaled<L, s>(r3, ux, uy, uz, Ux, Uy, Uz);
-        feq[s] = w[s] * fma_t(t, fma_t(t, h, 1.0f), A);
+        const T t = s == 0 ? T(0) : edot_scaled<L, s, STEP>(r3, ux, uy, uz, Ux, Uy, Uz);
+        feq[s] = w[s] * fma_t(t, fma_t(t, h, T(1)), A);
     });
 }
 
@@ -631,7 +643,10 @@ __device__ inline void equilibrium_f32(float (&feq)[L::Q], float dlt, float rho,
 // type-5 increment its w, and the bounce-back and inlet/outlet
 // reconstructions keep their form because a direction and its partner have
 // the same weight.
-template <class L, class T, bool SHIFT, bool COLLIDE, bool SC = false>
+// STEP: see equilibrium_dev.
+// SOLIDS false: a solid node takes part in the arithmetic (to no avail) and
+// keeps its f (node_settle).
+template <class L, class T, bool SHIFT, bool COLLIDE, bool SC = false, bool STEP = true, bool SOLIDS = true>
 __device__ inline bool node_prepare(T (&f)[L::Q], T (&feq)[L::Q], int t, T &rho, T &ux, T &uy,
                                     T &uz, const StepArgs &a, const T *__restrict__ uy_head,
                                     const T (&w)[L::Q], uint32_t g) {
@@ -670,7 +685,7 @@ __device__ inline bool node_prepare(T (&f)[L::Q], T (&feq)[L::Q], int t, T &rho,
             uz = mz / r;
         }
     }
-    if (t == 1) {
+    if (SOLIDS && t == 1) {
         // solid node: u = 0, whole-vector bounce-back, no relaxation
         // (TLBM_Partition.cpp:750-756, D3Q19LatticeStructure.hpp:65-76)
         ux = T(0); uy = T(0); uz = T(0);
@@ -700,7 +715,7 @@ __device__ inline bool node_prepare(T (&f)[L::Q], T (&feq)[L::Q], int t, T &rho,
         T inv_1mu = num<T>(a.inv_1mu, a.fl.inv_1mu), c_in = c_in0;
         if (a.inlet_uz) {
             // a prescribed inlet profile: 1/(1-u) and the deviation constant per node
-            const T u = T(a.inlet_uz[g % a.nxny]);
+            const T u = T(a.inlet_uz[g - udiv(g, a.div_nxny) * a.nxny]);
             uz = u;
             inv_1mu = T(1) / (T(1) - u);
             c_in = c_in0 + (u - num<T>(a.u_bc, a.fl.u_bc));
@@ -735,7 +750,7 @@ __device__ inline bool node_prepare(T (&f)[L::Q], T (&feq)[L::Q], int t, T &rho,
     if (uy_head && t == 5) {  // no lattice with this type takes the two-step pass, which has no uy_head
         // set_uz_bc (LatticeStructure.hpp:166-177); the y term reads uy of
         // node s of this step, as the reference's uy[spd] does
-        const T ubc = a.inlet_uz ? T(a.inlet_uz[g % a.nxny]) : num<T>(a.u_bc, a.fl.u_bc);
+        const T ubc = a.inlet_uz ? T(a.inlet_uz[g - udiv(g, a.div_nxny) * a.nxny]) : num<T>(a.u_bc, a.fl.u_bc);
         each<1, Q>([&](auto s) {
             T br = T(-0.0);
             if (L::ez[s] > 0) br += (ubc - uz); else if (L::ez[s] < 0) br -= (ubc - uz);
@@ -745,45 +760,31 @@ __device__ inline bool node_prepare(T (&f)[L::Q], T (&feq)[L::Q], int t, T &rho,
         });
     }
     // compute_equilibrium, LatticeStructure.hpp:92-103
-    if constexpr (SHIFT && !SC && sizeof(T) == 4) {
-        equilibrium_f32<L>(feq, dlt, rho, ux, uy, uz, w);
+    if constexpr (SHIFT && !SC) {
+        equilibrium_dev<L, STEP>(feq, dlt, rho, ux, uy, uz, w);
     } else {
-        const T usq = ux * ux + uy * uy + uz * uz;
         if constexpr (SHIFT) {
+            TLBM_ROUND_EACH
             // f_eq - w = w (delta + rho (cu + cu^2/2 - 3u^2/2)), cu = 3 e.u,
             // rewritten with t = e.(3 rho u) = rho cu:  w (A + t + t^2 / (2 rho)),
             // A = delta - 3/2 rho u^2 (the same polynomial, fewer operations)
-            const T A = dlt - T(1.5) * rho * usq;
-            T h;
-            if constexpr (sizeof(T) == 8)
-                h = T(0.5) / rho;  // FP32X: every operation in FP64
-            else
-                h = T(0.5) * __builtin_amdgcn_rcpf(rho);
-            // FP16 (SC): U = (3 + dt3) rho u, as fma(3 rho, u, dt3 rho u),
-            // which rounds the exact product plus the correction once, so
-            // the correction survives rounding on average (3 + dt3 itself
-            // rounds to 3).  The other storages have dt3 = 0 and form
-            // 3 rho u as a plain product, which leaves the compiler free to
-            // contract it into the sums of t below.
-            T Ux, Uy, Uz;
-            if constexpr (SC) {
-                const T r3 = T(3) * rho, rd = T(a.dt3) * rho;
-                Ux = fma_t(r3, ux, rd * ux);
-                Uy = fma_t(r3, uy, rd * uy);
-                Uz = fma_t(r3, uz, rd * uz);
-            } else {
-                const T t3 = T(3);
-                Ux = t3 * rho * ux;
-                Uy = t3 * rho * uy;
-                Uz = t3 * rho * uz;
-            }
+            const T usq = speed2<STEP>(ux, uy, uz);
+            const T A = fma_t(-(T(1.5) * rho), usq, dlt);
+            const T h = T(0.5) * __builtin_amdgcn_rcpf(rho);
+            // U = (3 + dt3) rho u, as fma(3 rho, u, dt3 rho u), which rounds
+            // the exact product plus the correction once, so the correction
+            // survives rounding on average (3 + dt3 itself rounds to 3).
+            const T r3 = T(3) * rho, rd = T(a.dt3) * rho;
+            const T Ux = fma_t(r3, ux, rd * ux);
+            const T Uy = fma_t(r3, uy, rd * uy);
+            const T Uz = fma_t(r3, uz, rd * uz);
             each<0, Q>([&](auto s) {
                 const T t = (s == 0) ? T(0) : edot<T>(L::ex[s], L::ey[s], L::ez[s], Ux, Uy, Uz);
-                feq[s] = SC ? A + t * (T(1) + t * h) : w[s] * (A + t * (T(1) + t * h));
+                feq[s] = fma_t(t, fma_t(t, h, T(1)), A);
             });
-            const T corr = rho * (T(1.5) * T(a.dk1) * usq - T(a.dk0));
-            feq[0] += SC ? corr * T(a.h_scale[0]) : corr;
+            feq[0] = fma_t(rho * fma_t(T(1.5) * T(a.dk1), usq, -T(a.dk0)), T(a.h_scale[0]), feq[0]);
         } else {
+            const T usq = ux * ux + uy * uy + uz * uz;
             each<0, Q>([&](auto s) {
                 const T cu = (s == 0) ? T(0) : T(3) * edot<T>(L::ex[s], L::ey[s], L::ez[s], ux, uy, uz);
                 feq[s] = w[s] * rho * (T(1) + cu + T(0.5) * (cu * cu) - T(1.5) * usq);
@@ -802,28 +803,78 @@ __device__ inline bool node_prepare(T (&f)[L::Q], T (&feq)[L::Q], int t, T &rho,
     return true;
 }
 
-// Non-equilibrium stress Pi = sum_s e e (f - feq) (compute_strain_tensor,
+// A pair of opposite directions s, bb[s] in the stress sum of axes A and B:
+// e_A e_B, and the n-th pair (by its first direction) that enters the sum.
+template <class L, int A, int B>
+constexpr int stress_sign(int s) {
+    const int e[3] = {L::ex[s], L::ey[s], L::ez[s]};
+    return e[A] * e[B];
+}
+template <class L, int A, int B>
+constexpr int stress_pair(int n) {
+    for (int s = 1;; ++s)
+        if (s < L::bb[s] && stress_sign<L, A, B>(s) != 0 && n-- == 0) return s;
+}
+
+// Sum of e_A e_B w v over the pairs, v[s] a pair's value, with every rounding
+// written out: each product enters unrounded, except that one of the first
+// two has to be rounded (ROUND_FIRST: the first).
+template <class L, int A, int B, bool ROUND_FIRST>
+__device__ inline float stress_sum(const float (&v)[L::Q], const float (&w)[L::Q]) {
+    TLBM_ROUND_EACH
+    constexpr int p = stress_pair<L, A, B>(0), q = stress_pair<L, A, B>(1);
+    static_assert(stress_sign<L, A, B>(p) > 0, "the first term enters as it is");
+    const float wq = stress_sign<L, A, B>(q) > 0 ? w[q] : -w[q];
+    float sum;
+    if constexpr (ROUND_FIRST) sum = fma_t(wq, v[q], w[p] * v[p]);
+    else sum = fma_t(w[p], v[p], wq * v[q]);
+    each<q + 1, L::Q>([&](auto s) {
+        constexpr int e = stress_sign<L, A, B>(s);
+        if constexpr (s < L::bb[s] && e != 0) sum = fma_t(e > 0 ? w[s] : -w[s], v[s], sum);
+    });
+    return sum;
+}
+
+// Non-equilibrium stress Pi = sum_s e e n, n = f - feq (compute_strain_tensor,
 // LatticeStructure.hpp:105-122): xx, yy, zz, xy, xz, yz.  SC: f and feq
 // hold h = d / w, and each difference is weighed by its w; a direction and
 // its partner (bounce-back table) have the same e e and the same w, so
 // their differences are added first and each pair enters a sum once (about
 // a third fewer operations than one term per direction).
 template <class L, class T, bool SC = false>
-__device__ inline void node_stress(const T (&f)[L::Q], const T (&feq)[L::Q], T (&pi)[6],
-                                   const T (&w)[L::Q]) {
-    T sxx = T(-0.0), syy = T(-0.0), szz = T(-0.0), sxy = T(-0.0), sxz = T(-0.0), syz = T(-0.0);
-    each<0, L::Q>([&](auto s) {
-        // the rest direction adds to no sum; the others come with their partner
-        if constexpr (SC && (s == 0 || L::bb[s] < s)) return;
-        const T fn = SC ? ((f[s] - feq[s]) + (f[L::bb[s]] - feq[L::bb[s]])) * w[s] : f[s] - feq[s];
-        if (L::ex[s] != 0) sxx += fn;
-        if (L::ey[s] != 0) syy += fn;
-        if (L::ez[s] != 0) szz += fn;
-        if (L::ex[s] * L::ey[s] > 0) sxy += fn; else if (L::ex[s] * L::ey[s] < 0) sxy -= fn;
-        if (L::ex[s] * L::ez[s] > 0) sxz += fn; else if (L::ex[s] * L::ez[s] < 0) sxz -= fn;
-        if (L::ey[s] * L::ez[s] > 0) syz += fn; else if (L::ey[s] * L::ez[s] < 0) syz -= fn;
-    });
-    pi[0] = sxx; pi[1] = syy; pi[2] = szz; pi[3] = sxy; pi[4] = sxz; pi[5] = syz;
+__device__ inline void node_stress(const T (&n)[L::Q], T (&pi)[6], const T (&w)[L::Q]) {
+    if constexpr (SC) {
+        T v[L::Q];
+        each<1, L::Q>([&](auto s) {  // the rest direction adds to no sum
+            if constexpr (s < L::bb[s]) v[s] = n[s] + n[L::bb[s]];
+        });
+        pi[0] = stress_sum<L, 0, 0, false>(v, w);
+        pi[1] = stress_sum<L, 1, 1, false>(v, w);
+        pi[2] = stress_sum<L, 2, 2, false>(v, w);
+        pi[3] = stress_sum<L, 0, 1, L::Q != 19>(v, w);
+        pi[4] = stress_sum<L, 0, 2, L::Q != 19>(v, w);
+        pi[5] = stress_sum<L, 1, 2, L::Q == 15>(v, w);
+    } else {
+        T sxx = T(-0.0), syy = T(-0.0), szz = T(-0.0), sxy = T(-0.0), sxz = T(-0.0), syz = T(-0.0);
+        each<0, L::Q>([&](auto s) {
+            const T fn = n[s];
+            if (L::ex[s] != 0) sxx += fn;
+            if (L::ey[s] != 0) syy += fn;
+            if (L::ez[s] != 0) szz += fn;
+            if (L::ex[s] * L::ey[s] > 0) sxy += fn; else if (L::ex[s] * L::ey[s] < 0) sxy -= fn;
+            if (L::ex[s] * L::ez[s] > 0) sxz += fn; else if (L::ex[s] * L::ez[s] < 0) sxz -= fn;
+            if (L::ey[s] * L::ez[s] > 0) syz += fn; else if (L::ey[s] * L::ez[s] < 0) syz -= fn;
+        });
+        pi[0] = sxx; pi[1] = syy; pi[2] = szz; pi[3] = sxy; pi[4] = sxz; pi[5] = syz;
+    }
+}
+
+// Pi : Pi with every rounding written out.
+template <class T>
+__device__ inline T stress_norm2(const T (&pi)[6]) {
+    TLBM_ROUND_EACH
+    return fma_t(T(2), fma_t(pi[5], pi[5], fma_t(pi[3], pi[3], pi[4] * pi[4])),
+                 fma_t(pi[2], pi[2], fma_t(pi[0], pi[0], pi[1] * pi[1])));
 }
 
 // |Pi| as apply_turbulence_model forms it (LatticeStructure.hpp:147).
@@ -836,40 +887,33 @@ __device__ inline T stress_norm(const T (&pi)[6]) {
 // apply_turbulence_model, LatticeStructure.hpp:140-153.  FAST (FP16
 // storage, whose own rounding is ~1e-3 of a population): the hardware square
 // roots and reciprocal, 1 ulp each, in place of the correctly rounded ones.
-template <class T, bool FAST = false>
+template <class T, bool FAST, bool SHIFT, bool STEP>
 __device__ inline T smagorinsky_omega(const T (&pi)[6], const StepArgs &a) {
+    const T cs = num<T>(a.cs, a.fl.cs), nu = num<T>(a.nu, a.fl.nu), nu2 = num<T>(a.nu2, a.fl.nu2);
     if constexpr (FAST) {
         static_assert(sizeof(T) == 4, "FP32 arithmetic");
-        const float n2 = pi[0] * pi[0] + pi[1] * pi[1] + pi[2] * pi[2] +
-                         2.f * (pi[3] * pi[3] + pi[4] * pi[4] + pi[5] * pi[5]);
-        const float P = __builtin_amdgcn_sqrtf(__builtin_amdgcn_sqrtf(n2) * a.fl.cs + a.fl.nu2) -
-                        a.fl.nu;
-        return __builtin_amdgcn_rcpf(3.f * (a.fl.nu + P * (1.f / 6.f)) + 0.5f);
-    }
-    if constexpr (sizeof(T) == 4) {
+        const T P = fma_t(__builtin_amdgcn_sqrtf(stress_norm2(pi)), cs, nu2);
+        const T nu_e = __builtin_amdgcn_sqrtf(P) - nu;
+        return __builtin_amdgcn_rcpf(fma_t(T(3), fma_t(nu_e, T(1.f / 6.f), nu), T(0.5)));
+    } else if constexpr (SHIFT) {
         TLBM_ROUND_EACH
-        const float n2 = fma_t(2.f, fma_t(pi[5], pi[5], fma_t(pi[3], pi[3], pi[4] * pi[4])),
-                               fma_t(pi[2], pi[2], fma_t(pi[1], pi[1], pi[0] * pi[0])));
-        const float P = sqrtf(fma_t(sqrtf(n2), a.fl.cs, a.fl.nu2)) - a.fl.nu;
-        return 1.f / fma_t(3.f, a.fl.nu + P / 6.f, 0.5f);
+        T n2 = stress_norm2(pi);
+        if constexpr (sizeof(T) == 4 && STEP)
+            n2 = fma_t(T(2), fma_t(pi[5], pi[5], fma_t(pi[3], pi[3], pi[4] * pi[4])),
+                       fma_t(pi[2], pi[2], fma_t(pi[1], pi[1], pi[0] * pi[0])));
+        const T P = sqrt(fma_t(sqrt(n2), cs, nu2)) - nu;
+        return T(1) / fma_t(T(3), nu + P / T(6), T(0.5));
+    } else {
+        T P = stress_norm<T>(pi);
+        P *= cs;
+        P = sqrt(P + nu2) - nu;
+        const T nu_e = P / T(6);
+        return T(1) / (T(3) * (nu + nu_e) + T(0.5));
     }
-    T P = stress_norm<T>(pi);
-    P *= num<T>(a.cs, a.fl.cs);
-    P = sqrt(P + num<T>(a.nu2, a.fl.nu2)) - num<T>(a.nu, a.fl.nu);
-    const T nu_e = P / T(6);
-    return T(1) / (T(3) * (num<T>(a.nu, a.fl.nu) + nu_e) + T(0.5));
 }
 
-// relax, LatticeStructure.hpp:155-163.
-template <class L, class T>
-__device__ inline void node_relax(T (&f)[L::Q], const T (&feq)[L::Q], T om) {
-    each<0, L::Q>([&](auto s) {
-        f[s] = f[s] - om * (f[s] - feq[s]);
-    });
-}
-
-// relax of a fluid node in FP32 storage, conserving to the rounding of
-// f - feq.  In exact arithmetic the mass and momentum of f - feq are small
+// n = f - feq of a fluid node in FP32 storage, made conserving to its rounding.
+// In exact arithmetic the mass and momentum of f - feq are small
 // values set by the weights (the reference's D3Q15/D3Q19 float weights do
 // not sum to 1); rounded FP32 equilibria miss them by a few ulp of feq, the
 // same amount at every node of a steady flow, and that residue accumulates
@@ -878,28 +922,25 @@ __device__ inline void node_relax(T (&f)[L::Q], const T (&feq)[L::Q], T om) {
 // float roundings: the D3Q27 weights sum to 1 in double but to 1 + 7.5e-9
 // in float, a mass source FP64 does not have.  The residue of mass m0 and
 // momentum m is taken out of f - feq as w_s (m0 + 3 e_s.m), which carries
-// that mass and momentum.
-template <class L>
-__device__ inline void node_relax_conserving(float (&f)[L::Q], const float (&feq)[L::Q],
-                                             const float (&w)[L::Q], float om, float rho,
-                                             float ux, float uy, float uz, const StepArgs &a) {
+// that mass and momentum.  Where fluid is false n stays.
+template <class L, bool STEP>
+__device__ inline void conserve(float (&n)[L::Q], const float (&w)[L::Q], bool fluid, float rho, float ux, float uy,
+                                float uz, const StepArgs &a) {
     TLBM_ROUND_EACH
     constexpr int Q = L::Q;
-    float nq[Q], m0 = -0.0f, mx = -0.0f, my = -0.0f, mz = -0.0f;
+    float m0 = -0.0f, mx = -0.0f, my = -0.0f, mz = -0.0f;
     each<0, Q>([&](auto s) {
         TLBM_ROUND_EACH
-        nq[s] = f[s] - feq[s];
-        m0 += nq[s];
-        if (L::ex[s] > 0) mx += nq[s]; else if (L::ex[s] < 0) mx -= nq[s];
-        if (L::ey[s] > 0) my += nq[s]; else if (L::ey[s] < 0) my -= nq[s];
-        if (L::ez[s] > 0) mz += nq[s]; else if (L::ez[s] < 0) mz -= nq[s];
+        m0 += n[s];
+        if (L::ex[s] > 0) mx += n[s]; else if (L::ex[s] < 0) mx -= n[s];
+        if (L::ey[s] > 0) my += n[s]; else if (L::ey[s] < 0) my -= n[s];
+        if (L::ez[s] > 0) mz += n[s]; else if (L::ez[s] < 0) mz -= n[s];
     });
-    const float usq = fma_t(uz, uz, fma_t(uy, uy, ux * ux));
-    m0 = fma_t(-rho, fma_t(1.5f * a.k1, usq, -a.k0), m0);
     const float rk = rho * a.k2;
-    mx = fma_t(-rk, ux, mx);
-    my = fma_t(-rk, uy, my);
-    mz = fma_t(-rk, uz, mz);
+    m0 = fluid ? fma_t(-rho, fma_t(1.5f * a.k1, speed2<STEP>(ux, uy, uz), -a.k0), m0) : 0.0f;
+    mx = fluid ? fma_t(-rk, ux, mx) : 0.0f;
+    my = fluid ? fma_t(-rk, uy, my) : 0.0f;
+    mz = fluid ? fma_t(-rk, uz, mz) : 0.0f;
     const float Mx = 3.0f * mx, My = 3.0f * my, Mz = 3.0f * mz;
     each<0, Q>([&](auto s) {
         TLBM_ROUND_EACH
@@ -908,8 +949,8 @@ __device__ inline void node_relax_conserving(float (&f)[L::Q], const float (&feq
         if constexpr (x * x + y * y + z * z == 1)
             c = fma_t(3.0f * float(x + y + z), x ? mx : y ? my : mz, m0);
         else if constexpr (s != 0)
-            c = m0 + edot_scaled<L, s>(3.0f, mx, my, mz, Mx, My, Mz);
-        f[s] = fma_t(-om, fma_t(-w[s], c, nq[s]), f[s]);
+            c = m0 + edot_scaled<L, s, STEP>(3.0f, mx, my, mz, Mx, My, Mz);
+        n[s] = fma_t(-w[s], c, n[s]);
     });
 }
 
@@ -921,318 +962,56 @@ __device__ inline void node_relax_conserving(float (&f)[L::Q], const float (&feq
 template <int ST, int Q>
 constexpr bool kConserve = ST == ST_F32;
 
-// 1/x to within rounding: in float the hardware reciprocal (1 ulp) and one
-// Newton step (3 operations; the correctly rounded division takes 10).
-__device__ inline double rcp_newton(double x) { return 1.0 / x; }
-__device__ inline float rcp_newton(float x) {
-    const float r = __builtin_amdgcn_rcpf(x);
-    return fma_t(r, fma_t(-x, r, 1.0f), r);
-}
-
-// ---- deviation storage: the node update by direction pairs ---------------------------------
-// A direction s and its opposite b = bb[s] have the same weight w and the
-// equilibria w (c + t) and w (c - t), c = A + t^2 h, so what a pair needs
-// comes from its sum and its difference: a fluid node's update takes about
-// 170 operations (D3Q19) where one direction at a time took 250.  n[] holds
-// f - feq in that form: n[0], and per pair (s < b) n[s] = n_s + n_b and
-// n[b] = n_s - n_b.  Node types other than fluid patch the fluid update
-// where a wavefront holds any (branches on the whole wavefront, so that a
-// lane's values are not kept for two sides of a branch).
-// SC: f[] and n[] hold h = d / w.
-
-// The inlet's (outlet's) unknown populations, those with e_z > 0 (< 0):
-// f_unknown = feq_unknown + f_partner - feq_partner, so the unknown's f - feq
-// is its partner's.  With the opposite direction for a partner (D3Q19, D3Q27)
-// the equilibria differ by 2 w t, with the mirror image in z (D3Q15) by
-// 2 w e_z U_z (1 + 2 h (e_x U_x + e_y U_y)).  Selects, no branches: where the
-// two sides of a branch name different elements of f, the compiler indexes
-// f by a variable, and f goes to memory or is copied whole.
-template <class L, class T, bool SC>
-__device__ inline void pairs_rebuild(T (&f)[L::Q], T (&n)[L::Q], bool inlet, bool outlet, T h, T Ux, T Uy, T Uz,
-                                     const T (&w)[L::Q]) {
-    constexpr bool kOpposite = L::in_par[1] == L::bb[L::in_unk[1]];
-    each<0, L::n_unk>([&](auto k) {
-        constexpr int s = L::in_unk[k], p = L::in_par[k];
-        const T w2 = SC ? T(2.0) : T(2.0) * w[s];
-        T d;  // feq_s - feq_p
-        if constexpr (kOpposite || L::ex[s] == 0)
-            d = w2 * edot<T>(L::ex[s], L::ey[s], L::ez[s], Ux, Uy, Uz);
-        else
-            d = w2 * Uz * fma_t(T(2.0) * h, edot<T>(L::ex[s], L::ey[s], 0, Ux, Uy, Uz), T(1.0));
-        const T fs = f[s], fp = f[p];
-        f[s] = inlet ? fp + d : fs;
-        f[p] = outlet ? fs - d : fp;
-    });
-    if constexpr (kOpposite) {
-        each<0, L::n_unk>([&](auto k) {
-            constexpr int s = L::in_unk[k], b = L::bb[s], lo = s < b ? s : b, hi = s < b ? b : s;
-            const T nb = s < b ? n[lo] - n[hi] : n[lo] + n[hi];  // 2 n_b
-            const T ns = s < b ? n[lo] + n[hi] : n[lo] - n[hi];  // 2 n_s
-            n[lo] = inlet ? nb : outlet ? ns : n[lo];
-            n[hi] = inlet || outlet ? T(0.0) : n[hi];
-        });
-    } else {
-        // D3Q15: the pairs (7, 14), (8, 13), (9, 12), (10, 11) trade members
-        // with the mirror images 7-11, 8-12, 9-13, 10-14; 5 and 6 are both
-        const T n5 = n[5] + n[6], n6 = n[5] - n[6];
-        n[5] = inlet ? n6 : outlet ? n5 : n[5];
-        n[6] = inlet || outlet ? T(0.0) : n[6];
-        each<7, 9>([&](auto k) {
-            // two pairs at a time: (s, b) and (m, q), q the mirror of s, m that of b
-            constexpr int s = k, b = L::bb[s], q = s + 4, m = L::bb[q];
-            const T xs = T(0.5) * (n[s] + n[b]), xb = T(0.5) * (n[s] - n[b]);
-            const T xm = T(0.5) * (n[m] + n[q]), xq = T(0.5) * (n[m] - n[q]);
-            const T ys = inlet ? xq : xs, ym = inlet ? xb : xm;
-            const T yb = outlet ? xm : xb, yq = outlet ? xs : xq;
-            n[s] = ys + yb;
-            n[b] = ys - yb;
-            n[m] = ym + yq;
-            n[q] = ym - yq;
-        });
-    }
-}
-
-// The step's rules up to f - feq (node_prepare's): moments, the inlet,
-// outlet and type-5 rules, equilibrium, reconstruction; fills n[].  A solid
-// node's n is finite (it takes no part in the rules).
-// CONSERVE: the rounding residue of mass and momentum in a fluid node's
-// f - feq is taken out.  In exact arithmetic f - feq has the mass and
-// momentum that the weights w set (the reference's D3Q15/D3Q19 T weights
-// do not sum to 1); rounded FP32 equilibria miss them by a few ulp of feq,
-// the same amount at every node of a steady flow, and that residue would
-// accumulate step after step (D3Q19 cylinder array: velocity L2 against FP64
-// 1.6e-5 after 20000 steps).  The targets are those of the weights w, not of
-// their T roundings: the D3Q27 weights sum to 1 in double but to
-// 1 + 7.5e-9 in float, a mass source FP64 does not have.  The residue is
-// measured on f - feq, whose own rounding is far below that of feq, and mass
-// m0 and momentum m of it are taken out as w_s (m0 + 3 e_s.m).  (The mass out
-// of the rest population and the momentum out of the axis pairs alone would
-// be 0.5 % (D3Q19) to 2 % (D3Q27) faster and as accurate, but not isotropic.)
-// The rounding of a steady FP32 flow's moments repeats every step, so every
-// operation is written out (TLBM_ROUND_EACH: products and sums are contracted
-// only where fma_t says so): both step kernels then give the same bits, and
-// the drift that tests bound is that of this source.  Of the equivalent forms
-// of the equilibrium A + t (t h +- 1) keeps a uniform flow's momentum closest
-// to FP64's (D3Q19 float weights, 4000 steps: 4e-7; A + t^2 h +- t 1 to 5e-6).
-template <class L, class T, bool SC, bool CONSERVE>
-__device__ inline void pairs_prepare(T (&f)[L::Q], T (&n)[L::Q], int t, const StepArgs &a,
-                                     const T *__restrict__ uy_head, const T (&w)[L::Q], uint32_t g) {
-    TLBM_ROUND_EACH
-    static_assert(!(SC && CONSERVE), "the conserving form works on d");
-    T r = SC ? w[0] * f[0] : f[0], mx = T(-0.0), my = T(-0.0), mz = T(-0.0);
-    each_pair<L>([&](auto k) {
-        constexpr int s = k, b = L::bb[s];
-        n[s] = f[s] + f[b];
-        n[b] = f[s] - f[b];
-        if (SC) {
-            r = fma_t(w[s], n[s], r);
-            if (L::ex[s]) mx = fma_t(T(L::ex[s]) * w[s], n[b], mx);
-            if (L::ey[s]) my = fma_t(T(L::ey[s]) * w[s], n[b], my);
-            if (L::ez[s]) mz = fma_t(T(L::ez[s]) * w[s], n[b], mz);
-        } else {
-            r += n[s];
-            if (L::ex[s] > 0) mx += n[b]; else if (L::ex[s] < 0) mx -= n[b];
-            if (L::ey[s] > 0) my += n[b]; else if (L::ey[s] < 0) my -= n[b];
-            if (L::ez[s] > 0) mz += n[b]; else if (L::ez[s] < 0) mz -= n[b];
-        }
-    });
-    T dlt = r + num<T>(a.dw_d, a.dw), rho = T(1.0) + dlt;
-    T inv = t == 1 ? T(1.0) : rcp_newton(rho);
-    const bool inlet = t == 2, outlet = t == 3, ends = __any(inlet || outlet);
-    if (ends) {
-        // set_inletW_bc_macro, set_outletE_bc_macro
-        // (D3Q19LatticeStructure.hpp:108-156); at the outlet u_x and u_y of
-        // the node's own density are kept
-        T level = T(-0.0), in = T(-0.0), out = T(-0.0);
-        each<0, L::n_zero>([&](auto k) {
-            constexpr int s = L::zero_list[k];
-            level = SC ? fma_t(w[s], f[s], level) : level + f[s];
-        });
-        each<0, L::n_unk>([&](auto k) {
-            constexpr int s = L::in_list[k], p = L::out_list[k];
-            in = SC ? fma_t(w[s], f[s], in) : in + f[s];
-            out = SC ? fma_t(w[p], f[p], out) : out + f[p];
-        });
-        const T u_bc = num<T>(a.u_bc, a.fl.u_bc), rho_bc = num<T>(a.rho_bc, a.fl.rho_bc),
-                inv_bc = num<T>(a.inv_rho_bc, a.fl.inv_rho_bc), c_out = num<T>(a.c_out_d, a.c_out);
-        T uz = u_bc, inv_1mu = num<T>(a.inv_1mu, a.fl.inv_1mu), c_in = num<T>(a.c_in_d, a.c_in);
-        if (a.inlet_uz) {
-            // a prescribed inlet profile: 1/(1-u) and the deviation constant per node
-            uz = T(a.inlet_uz[g % a.nxny]);
-            inv_1mu = T(1.0) / (T(1.0) - uz);
-            c_in += uz - u_bc;
-        }
-        const T keep = inlet ? T(0.0) : outlet ? rho_bc * inv : T(1.0);
-        dlt = inlet ? inv_1mu * (c_in + (T(2.0) * in + level)) : outlet ? num<T>(a.rho_bc - 1.0, a.drho_bc) : dlt;
-        rho = outlet ? rho_bc : T(1.0) + dlt;
-        inv = outlet ? inv_bc : inlet ? rcp_newton(rho) : inv;
-        mx *= keep;
-        my *= keep;
-        mz = inlet ? rho * uz : outlet ? rho_bc * (inv_bc * (c_out + (T(2.0) * out + level))) : mz;
-    }
-    // rho u^2 from rounded squares, as node_prepare forms it
-    const T q2 = inv * (mx * mx + my * my + mz * mz);
-    const T h = T(0.5) * inv, A = fma_t(T(-1.5), q2, dlt);
-    // FP16 (SC): 3 + dt3 times the momentum, rounded once, so that the
-    // correction (which 3 + dt3 would lose) survives rounding on average
-    const T Ux = SC ? fma_t(T(3.0), mx, T(a.dt3) * mx) : T(3.0) * mx;
-    const T Uy = SC ? fma_t(T(3.0), my, T(a.dt3) * my) : T(3.0) * my;
-    const T Uz = SC ? fma_t(T(3.0), mz, T(a.dt3) * mz) : T(3.0) * mz;
-    n[0] = SC ? f[0] - A : fma_t(-w[0], A, f[0]);
-    if (SC) n[0] -= (T(1.5) * T(a.dk1) * q2 - T(a.dk0) * rho) * T(a.h_scale[0]);
-    T m0 = n[0], cx = T(-0.0), cy = T(-0.0), cz = T(-0.0);
-    each_pair<L>([&](auto k) {
-        TLBM_ROUND_EACH
-        constexpr int s = k, b = L::bb[s];
-        const T tt = edot<T>(L::ex[s], L::ey[s], L::ez[s], Ux, Uy, Uz);
-        if (CONSERVE) {
-            // each direction's f - feq rounds once, far below f; formed from
-            // the pair's sum and difference it would carry their rounding
-            const T x = fma_t(-w[s], fma_t(tt, fma_t(tt, h, T(1.0)), A), f[s]);
-            const T y = fma_t(-w[s], fma_t(tt, fma_t(tt, h, T(-1.0)), A), f[b]);
-            n[s] = x + y;
-            n[b] = x - y;
-            m0 += n[s];
-            if (L::ex[s] > 0) cx += n[b]; else if (L::ex[s] < 0) cx -= n[b];
-            if (L::ey[s] > 0) cy += n[b]; else if (L::ey[s] < 0) cy -= n[b];
-            if (L::ez[s] > 0) cz += n[b]; else if (L::ez[s] < 0) cz -= n[b];
-        } else {
-            const T c = fma_t(tt * tt, h, A);
-            const T w2 = SC ? T(2.0) : T(2.0) * w[s];
-            n[s] = fma_t(-w2, c, n[s]);
-            n[b] = fma_t(-w2, tt, n[b]);
-        }
-    });
-    if constexpr (CONSERVE) {
-        const bool fluid = t == 0;
-        m0 = fluid ? m0 - fma_t(T(1.5) * T(a.k1), q2, -(T(a.k0) * rho)) : T(0.0);
-        cx = fluid ? T(3.0) * fma_t(-T(a.k2), mx, cx) : T(0.0);
-        cy = fluid ? T(3.0) * fma_t(-T(a.k2), my, cy) : T(0.0);
-        cz = fluid ? T(3.0) * fma_t(-T(a.k2), mz, cz) : T(0.0);
-        n[0] = fma_t(-w[0], m0, n[0]);
-        each_pair<L>([&](auto k) {
-            TLBM_ROUND_EACH
-            constexpr int s = k, b = L::bb[s];
-            const T w2 = T(2.0) * w[s];
-            n[s] = fma_t(-w2, m0, n[s]);
-            n[b] = fma_t(-w2, edot<T>(L::ex[s], L::ey[s], L::ez[s], cx, cy, cz), n[b]);
-        });
-    }
-    if (ends) pairs_rebuild<L, T, SC>(f, n, inlet, outlet, h, Ux, Uy, Uz, w);
-    if (uy_head && __any(t == 5)) {
-        // set_uz_bc (LatticeStructure.hpp:166-177); the y term reads uy of
-        // node s of this step, as the reference's uy[spd] does
-        const T ubc = a.inlet_uz ? T(a.inlet_uz[g % a.nxny]) : num<T>(a.u_bc, a.fl.u_bc);
-        const T ux = mx * inv, uz = mz * inv, r3 = t == 5 ? T(3.0) * rho : T(0.0);
-        each_pair<L>([&](auto k) {
-            constexpr int s = k, b = L::bb[s];
-            T in[2];
-            each<0, 2>([&](auto i) {
-                constexpr int d = i ? b : s;
-                T br = T(-0.0);
-                if (L::ez[d] > 0) br += (ubc - uz); else if (L::ez[d] < 0) br -= (ubc - uz);
-                if (L::ex[d] > 0) br -= ux; else if (L::ex[d] < 0) br += ux;
-                if (L::ey[d] > 0) br -= uy_head[d]; else if (L::ey[d] < 0) br += uy_head[d];
-                in[i] = (SC ? r3 : r3 * w[s]) * br;
-                f[d] += in[i];
-            });
-            n[s] += in[0] + in[1];
-            n[b] += in[0] - in[1];
-        });
-    }
-}
-
-// Pi of a node from the pair sums of n[] (see node_stress).
-template <class L, class T, bool SC>
-__device__ inline void pair_stress(const T (&n)[L::Q], T (&pi)[6], const T (&w)[L::Q]) {
-#pragma unroll
-    for (int k = 0; k < 6; ++k) pi[k] = T(-0.0);
-    each_pair<L>([&](auto k) {
-        constexpr int s = k;
-        const T v = SC ? n[s] * w[s] : n[s];
-        if (L::ex[s] != 0) pi[0] += v;
-        if (L::ey[s] != 0) pi[1] += v;
-        if (L::ez[s] != 0) pi[2] += v;
-        if (L::ex[s] * L::ey[s] > 0) pi[3] += v; else if (L::ex[s] * L::ey[s] < 0) pi[3] -= v;
-        if (L::ex[s] * L::ez[s] > 0) pi[4] += v; else if (L::ex[s] * L::ez[s] < 0) pi[4] -= v;
-        if (L::ey[s] * L::ez[s] > 0) pi[5] += v; else if (L::ey[s] * L::ez[s] < 0) pi[5] -= v;
-    });
-}
-
-// Relaxation from n[] at rate om, and the solid node's whole-vector
-// bounce-back without relaxation (TLBM_Partition.cpp:750-756,
-// D3Q19LatticeStructure.hpp:65-76): rate 0, and the pairs trade places.
-// solids: the wavefront's solid lanes, __ballot(t == 1) (scalar registers, so
-// that the node type need not stay in a vector register until here).
+// Relaxation of a deviation storage's node from n = f - feq at rate om, and
+// the solid node's whole-vector bounce-back without relaxation
+// (TLBM_Partition.cpp:750-756, D3Q19LatticeStructure.hpp:65-76): a rate and an
+// n of 0 leave its f as it is, whatever it holds, and the pairs trade places.
+// Branches on the whole wavefront, each without another side: where two sides
+// leave a whole f, the compiler copies it.
 template <class L, class T>
-__device__ inline void pairs_relax(T (&f)[L::Q], const T (&n)[L::Q], uint64_t solids, T om, const StepArgs &a) {
-    const bool solid = __builtin_amdgcn_inverse_ballot_w64(solids);
-    om = solid || a.dynamics != 1 ? T(0.0) : om;
-    const T half = T(-0.5) * om;
-    f[0] = fma_t(-om, n[0], f[0]);
-    each_pair<L>([&](auto k) {
-        constexpr int s = k, b = L::bb[s];
-        f[s] = fma_t(half, n[s] + n[b], f[s]);
-        f[b] = fma_t(half, n[s] - n[b], f[b]);
-    });
+__device__ inline void node_settle(T (&f)[L::Q], T (&n)[L::Q], bool solid, T om, const StepArgs &a) {
+    const bool solids = __any(solid);
     if (solids) {
-        each_pair<L>([&](auto k) {
-            constexpr int s = k, b = L::bb[s];
-            const T x = f[s];
-            f[s] = solid ? f[b] : x;
-            f[b] = solid ? x : f[b];
+        om = solid ? T(0) : om;
+        each<0, L::Q>([&](auto s) { n[s] = solid ? T(0) : n[s]; });
+    }
+    if (a.dynamics == 1) each<0, L::Q>([&](auto s) { f[s] = fma_t(-om, n[s], f[s]); });
+    if (solids) {
+        each<1, L::Q>([&](auto s) {
+            if constexpr (s < L::bb[s]) {
+                const T x = f[s];
+                f[s] = solid ? f[L::bb[s]] : x;
+                f[L::bb[s]] = solid ? x : f[L::bb[s]];
+            }
         });
     }
 }
-
-// Deviation storages update their nodes by direction pairs, except FP32 D3Q15
-// and D3Q19 without the network, which go direction by direction
-// (equilibrium_f32, node_relax_conserving).  Both forms are as accurate, but
-// tau near 1/2 grows the difference of two roundings by orders of magnitude in
-// a few hundred steps, so a form is kept where it costs little: D3Q19
-// 128x128x512 154 against 145 us per step by pairs (165 against 149 with
-// Smagorinsky), D3Q15 125 against 118.  D3Q27 goes by pairs: 207 against 254 us
-// (192^3, Smagorinsky), whose registers leave no room for the other form.
-template <int ST, int Q>
-constexpr bool kPairForm = !(ST == ST_F32 && Q != 27);
 
 // The whole reference update of one node (TLBM_Partition.cpp:742-807).
 // CONSERVE: fluid nodes relax conserving.  SC: the scaled form of node_prepare
-// (the relaxation is the same in either scale).  PAIRS: by direction pairs.
-template <class L, class T, bool SHIFT, bool COLLIDE, bool CONSERVE = false, bool SC = false, bool PAIRS = true>
+// (the relaxation is the same in either scale).
+template <class L, class T, bool SHIFT, bool COLLIDE, bool CONSERVE = false, bool SC = false>
 __device__ inline void node_update(T (&f)[L::Q], int t, T &rho, T &ux, T &uy, T &uz,
                                    const StepArgs &a, const T *__restrict__ uy_head,
                                    const T (&w)[L::Q], uint32_t g) {
     static_assert(!(SC && CONSERVE), "the conserving relax works on d");
-    if constexpr (COLLIDE && SHIFT && PAIRS) {
-        T n[L::Q], om = num<T>(a.omega, a.fl.omega);
-        const uint64_t solids = __ballot(t == 1);
-        pairs_prepare<L, T, SC, CONSERVE>(f, n, t, a, uy_head, w, g);
-        if (a.smag) {
-            T pi[6];
-            pair_stress<L, T, SC>(n, pi, w);
-            om = smagorinsky_omega<T, SC>(pi, a);
-        }
-        pairs_relax<L, T>(f, n, solids, om, a);
-        return;
-    }
     T feq[L::Q];
-    if (!node_prepare<L, T, SHIFT, COLLIDE, SC>(f, feq, t, rho, ux, uy, uz, a, uy_head, w, g)) return;
+    const bool relaxes = node_prepare<L, T, SHIFT, COLLIDE, SC, true, !(SHIFT && COLLIDE)>(f, feq, t, rho, ux, uy, uz, a, uy_head, w, g);
     if (!COLLIDE) return;
-    T om = num<T>(a.omega, a.fl.omega);
+    if (!SHIFT && !relaxes) return;
+    T n[L::Q], om = num<T>(a.omega, a.fl.omega);
+    each<0, L::Q>([&](auto s) { n[s] = f[s] - feq[s]; });
     if (a.smag) {
         T pi[6];
-        node_stress<L, T, SC>(f, feq, pi, w);
-        om = smagorinsky_omega<T, SC>(pi, a);
+        node_stress<L, T, SC>(n, pi, w);
+        om = smagorinsky_omega<T, SC, SHIFT, true>(pi, a);
     }
-    if (a.dynamics == 1) {
-        if constexpr (CONSERVE) {
-            if (t == 0) {
-                node_relax_conserving<L>(f, feq, w, om, rho, ux, uy, uz, a);
-                return;
-            }
-        }
-        node_relax<L, T>(f, feq, om);
+    if constexpr (SHIFT) {
+        if constexpr (CONSERVE) conserve<L, true>(n, w, t == 0, rho, ux, uy, uz, a);
+        node_settle<L>(f, n, t == 1, om, a);
+    } else if (a.dynamics == 1) {
+        // relax, LatticeStructure.hpp:155-163
+        each<0, L::Q>([&](auto s) { f[s] = f[s] - om * n[s]; });
     }
 }
 
@@ -1271,8 +1050,7 @@ template <class L, int ST, int MODE, bool REMAP = true, bool NTLOAD = false, boo
           int BS = kBlock>
 __global__ void __launch_bounds__(BS)
 __attribute__((amdgpu_waves_per_eu(
-    MODE == MODE_STEP || MODE == MODE_STEP_SMALL ? kStepWaves<ST, L::Q> : 1,
-    MODE == MODE_STEP || MODE == MODE_STEP_SMALL ? kStepWavesMax<ST, L::Q> : 8)))
+    1, MODE == MODE_STEP || MODE == MODE_STEP_SMALL ? kStepWavesMax<ST, L::Q> : 8)))
 k_lbm(const typename StorageT<ST>::st *__restrict__ fin, typename StorageT<ST>::st *__restrict__ fout,
       const uint8_t *__restrict__ nd_type, const uint8_t *__restrict__ chunk_type,
       void *__restrict__ out, const typename StorageT<ST>::T *__restrict__ uy_head, StepArgs a) {
@@ -1334,7 +1112,7 @@ k_lbm(const typename StorageT<ST>::st *__restrict__ fin, typename StorageT<ST>::
             sum[2 * n] = s2 + double(uz);
             sum[3 * n] = s3 + double(rho);
         }
-        node_update<L, T, S::kShift, true, kConserve<ST, Q>, S::kScaled, kPairForm<ST, Q>>(
+        node_update<L, T, S::kShift, true, kConserve<ST, Q>, S::kScaled>(
             f, t, rho, ux, uy, uz, a, uy_head, w, g);
         const PushOut<L, ST> po(fout, (blk * BS) >> StorageT<ST>::kCB, g);
         const uint32_t rs = ST == ST_F16 ? round_stream(g, a.step) : 0u;
@@ -1342,11 +1120,12 @@ k_lbm(const typename StorageT<ST>::st *__restrict__ fin, typename StorageT<ST>::
     } else if constexpr (MODE == MODE_STRESS) {
         T feq[Q], pi[6] = {T(0), T(0), T(0), T(0), T(0), T(0)};
         T c = T(0);
-        if (node_prepare<L, T, S::kShift, true, S::kScaled>(f, feq, t, rho, ux, uy, uz, a, uy_head,
+        if (node_prepare<L, T, S::kShift, true, S::kScaled, false>(f, feq, t, rho, ux, uy, uz, a, uy_head,
                                                             w, g) &&
             a.dynamics == 1) {
-            node_stress<L, T, S::kScaled>(f, feq, pi, w);
-            const T om = a.smag ? smagorinsky_omega<T>(pi, a) : num<T>(a.omega, a.fl.omega);
+            each<0, Q>([&](auto s) { feq[s] = f[s] - feq[s]; });
+            node_stress<L, T, S::kScaled>(feq, pi, w);
+            const T om = a.smag ? smagorinsky_omega<T, false, S::kShift, false>(pi, a) : num<T>(a.omega, a.fl.omega);
             c = T(0.5) * om - T(1);
         }
         T *macro = static_cast<T *>(out);
@@ -1376,31 +1155,35 @@ k_lbm(const typename StorageT<ST>::st *__restrict__ fin, typename StorageT<ST>::
     }
 }
 
+// The value is in its register at this point of the program.
+__device__ inline void formed_here(float &v) { __asm__ volatile("" : "+v"(v)); }
+
 // The update of a node whose relaxation time is the network's (mlp.h).  Every
 // lane of the wavefront takes part.  ready() is called once before the network
-// reads m (the workgroup's copy of the weights).  A solid node's result is
-// not used.
+// reads m (the workgroup's copy of the weights).
 template <class L, int ST, class F>
 __device__ inline void network_update(float (&f)[L::Q], int t, const StepArgs &a, const float *__restrict__ uy_head,
                                       const float (&w)[L::Q], uint32_t g, const MlpPacked *m, F ready) {
     using S = StorageT<ST>;
-    float n[L::Q], pi[6];
-    const uint64_t solids = __ballot(t == 1);
-    pairs_prepare<L, float, S::kScaled, kConserve<ST, L::Q>>(f, n, t, a, uy_head, w, g);
-    // formed here, not sunk past the network with its three operands (registers)
-    __asm__ volatile("" : "+v"(n[0]));
-    pair_stress<L, float, S::kScaled>(n, pi, w);
+    const uint64_t solids = __ballot(t == 1);  // scalar registers: t is not held through the network
+    float n[L::Q], rho, ux, uy, uz, pi[6];  // n: f_eq, then f - f_eq
+    node_prepare<L, float, S::kShift, true, S::kScaled, false, false>(f, n, t, rho, ux, uy, uz, a, uy_head, w, g);
+    each<0, L::Q>([&](auto s) { n[s] = f[s] - n[s]; });
+    node_stress<L, float, S::kScaled>(n, pi, w);
     float feat[kMlpIn];
 #pragma unroll
     for (int k = 0; k < 6; ++k) feat[k] = pi[k] * a.cl_in;
     // the norm feature is rounded to bf16: the hardware square root (1 ulp) suffices
-    feat[6] = __builtin_amdgcn_sqrtf(pi[0] * pi[0] + pi[1] * pi[1] + pi[2] * pi[2] +
-                                     2.0f * (pi[3] * pi[3] + pi[4] * pi[4] + pi[5] * pi[5])) *
-              a.cl_in;
+    feat[6] = __builtin_amdgcn_sqrtf(stress_norm2(pi)) * a.cl_in;
+    // ahead of the network, so that rho, u and the operands of n are not held through it
+    if constexpr (kConserve<ST, L::Q>) {
+        conserve<L, false>(n, w, t == 0, rho, ux, uy, uz, a);
+        each<0, L::Q>([&](auto s) { formed_here(n[s]); });
+    }
     ready();
     const float zz = mlp_wave(feat, m);
     const float om = __builtin_amdgcn_rcpf(a.tau0 + a.cl_out * softplus_f(zz));  // 1 ulp
-    pairs_relax<L, float>(f, n, solids, om, a);
+    node_settle<L>(f, n, __builtin_amdgcn_inverse_ballot_w64(solids), om, a);
 }
 
 // This thread's share of copying the network's weights to LDS, by direct

@@ -206,7 +206,7 @@ k_lbm_pair(const typename StorageT<ST>::st *__restrict__ fin, typename StorageT<
             network_update<L, ST>(f, t, a, nullptr, w, g, &smlp, [] {});
         } else {
             T rho, ux, uy, uz;
-            node_update<L, T, S::kShift, true, kConserve<ST, Q>, S::kScaled, kPairForm<ST, Q>>(f, t, rho, ux, uy, uz, a, nullptr, w, g);
+            node_update<L, T, S::kShift, true, kConserve<ST, Q>, S::kScaled>(f, t, rho, ux, uy, uz, a, nullptr, w, g);
         }
     };
     int tn, tp = 0;
