@@ -50,10 +50,8 @@ std::mutex g_mu;
 Ring *g_kept[kKept] = {};
 int g_users = 0;
 
-hipError_t take(Ring **out) {
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return e;
+// A ring of device dev, which need not be the calling thread's.
+hipError_t take(int dev, Ring **out) {
     {
         std::lock_guard<std::mutex> lock(g_mu);
         for (Ring *&k : g_kept)
@@ -64,7 +62,11 @@ hipError_t take(Ring **out) {
     }
     Ring *r = new (std::nothrow) Ring;
     if (!r) return hipErrorOutOfMemory;
-    e = r->create(dev);
+    int was = dev;
+    hipError_t e = hipGetDevice(&was);
+    if (e == hipSuccess) e = hipSetDevice(dev);
+    if (e == hipSuccess) e = r->create(dev);
+    (void)hipSetDevice(was);
     if (e != hipSuccess) {
         delete r;
         return e;
@@ -224,7 +226,7 @@ hipError_t direct(const tlbm::CopyPart *parts, int n, bool widen, hipStream_t st
 
 namespace tlbm {
 
-hipError_t copy_to_host(const CopyPart *parts, int n, bool widen, hipStream_t stream) {
+hipError_t copy_to_host(const CopyPart *parts, int n, bool widen, hipStream_t stream, int device) {
     try {
         const size_t esz = widen ? sizeof(float) : sizeof(double);
         size_t bytes = 0;
@@ -232,7 +234,7 @@ hipError_t copy_to_host(const CopyPart *parts, int n, bool widen, hipStream_t st
         if (bytes >= (widen ? kRingFrom32 : kRingFrom64)) {
             Ring *taken = nullptr;
             // no pinned memory left, or no thread: the direct copy
-            if (take(&taken) == hipSuccess) {
+            if (take(device, &taken) == hipSuccess) {
                 const std::unique_ptr<Ring, void (*)(Ring *)> ring(taken, give);
                 hipError_t e = hipSuccess;
                 if (Copier(*ring, chunks_of(parts, n, esz), stream, widen).run(e)) return e;

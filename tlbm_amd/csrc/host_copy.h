@@ -26,8 +26,9 @@ struct CopyPart {
     size_t count;
 };
 
-// Copies n parts in stream order and returns when the host has the values.
-hipError_t copy_to_host(const CopyPart *parts, int n, bool widen, hipStream_t stream);
+// Copies n parts in the order of a stream of `device` and returns when the
+// host has the values.  The calling thread's device does not matter.
+hipError_t copy_to_host(const CopyPart *parts, int n, bool widen, hipStream_t stream, int device);
 
 // Rings are kept while any lattice is alive (at most two, of 8 MiB) and given
 // back with the last one.

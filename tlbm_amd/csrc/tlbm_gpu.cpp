@@ -156,6 +156,7 @@ struct tlbm_gpu {
     double *partial = nullptr;  // reduction partials
     int nparts = 0;
     bool has_lid = false;
+    int device = 0;       // of the stream and every buffer
     bool copies = false;  // holds a share of the host copy rings
     long long steps_since_set = 0;
     uint64_t step_count = 0;  // steps since creation (FP16 rounding stream)
@@ -316,9 +317,9 @@ int tlbm_gpu_create(const tlbm_params *p, const uint8_t *nd_type, tlbm_gpu **out
     };
     if (int rc = fixed_partials(&h->fixed_partial)) return cleanup_fail(rc);
     {
-        int dev = 0, cus = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        int cus = 0;
+        if (hipGetDevice(&h->device) != hipSuccess ||
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device) != hipSuccess)
             cus = 0;
         for (int net = 0; net < 2; ++net)
             h->pair[net] = !has_lid && cus > 0 && (net == 0 || p->storage == TLBM_STORAGE_F32) &&
@@ -484,7 +485,7 @@ static int download_planes(tlbm_gpu *h, const void *src, size_t count, bool comp
     int n = 0;
     for (int k = 0; k < nplanes; ++k)
         if (dst[k]) parts[n++] = {static_cast<const char *>(src) + size_t(k) * count * esz, dst[k], count};
-    TLBM_HIP(tlbm::copy_to_host(parts, n, esz == 4, h->stream));
+    TLBM_HIP(tlbm::copy_to_host(parts, n, esz == 4, h->stream, h->device));
     return TLBM_OK;
 }
 
