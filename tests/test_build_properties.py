@@ -213,3 +213,14 @@ def test_two_step_pass_has_no_lid_rule(code):
     global, buffer or LDS accesses) are not in the kernels."""
     for name, ins in _pair(code).items():
         assert not [x for x in ins if x.startswith("flat_load")], name
+
+
+def test_two_step_pass_waits_for_the_next_plane_in_full(code):
+    """The next plane's direct loads into LDS are waited for in full, ahead of
+    the stores.  A counted wait after the stores would hold only as long as
+    each of them stays behind the loads as one instruction of its own."""
+    for name, ins in _pair(code).items():
+        waits = [re.search(r"vmcnt\((\d+)\)", x) for x in ins if x.startswith("s_waitcnt")]
+        assert {m.group(1) for m in waits if m} == {"0"}, name
+        first = _first(ins, r"buffer_store")
+        assert any("vmcnt(0)" in x for x in ins[first - 80:first]), name

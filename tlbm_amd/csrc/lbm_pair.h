@@ -76,11 +76,8 @@ template <class L> struct PairShapes<L, ST_F32X> {
     using T1 = PairTile<L, ST_F32X, 32, L::Q == 27 ? 12 : 20>;
 };
 
-// s_waitcnt vmcnt(n), other counters free.
-template <int N>
-__device__ inline void wait_vmcnt() {
-    __builtin_amdgcn_s_waitcnt((N & 15) | 0x0F70 | ((N >> 4) << 14));
-}
+// s_waitcnt vmcnt(0), other counters free: every load and store sent has landed.
+__device__ inline void wait_vmcnt() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
 // The workgroup's barrier for LDS traffic: this wavefront's LDS accesses are
 // done before it (global loads and stores stay in flight).
@@ -113,7 +110,10 @@ k_lbm_pair(const typename StorageT<ST>::st *__restrict__ fin, typename StorageT<
     __shared__ alignas(16) st lds[TL::kStage + TL::NS * W * H];
     st *const stage = lds, *const swap = lds + TL::kStage;
     __shared__ std::conditional_t<NET, MlpPacked, int> smlp;
-    if constexpr (NET) stage_network(a.mlp, &smlp);
+    if constexpr (NET) {
+        static_assert(sizeof(MlpPacked) <= 16u * BS, "one 16-byte load per lane");
+        stage_network(a.mlp, &smlp);
+    }
 
     const uint32_t b = xcd_block(blockIdx.x, gridDim.x);
     const uint32_t seg = udiv(b, pl.div_tiles);
@@ -212,7 +212,7 @@ k_lbm_pair(const typename StorageT<ST>::st *__restrict__ fin, typename StorageT<
     int tn, tp = 0;
     load_plane(z0 - 1);
     tn = nd_type[wrapz(z0 - 1) * a.nxny + gxy];
-    wait_vmcnt<0>();
+    wait_vmcnt();
     for (int p = z0 - 1; p <= z1; ++p) {
         lds_barrier();  // plane p is staged; the last exchange has been read
         T f[Q];
@@ -254,22 +254,22 @@ k_lbm_pair(const typename StorageT<ST>::st *__restrict__ fin, typename StorageT<
                 const __amdgpu_buffer_rsrc_t rsrc = make_rsrc(uintptr_t(fout) + back, a.fbytes - back);
                 const uint32_t r = gxy + (first - c * CH);
                 const uint32_t off = (r + __umul24(r >> CB, (Q - 1) * CH)) * kSize;
+                wait_vmcnt();  // plane p + 1 has landed (ahead of the stores, which then need no count)
                 if (own) {
                     each<0, Q>([&](auto s) {
                         RawBuf<st>::template store<kAuxNT>(S::step_out(f[s], s, a, rs + uint32_t(s) * kStreamStep),
                                                            rsrc, off, uint32_t(s) * CH * kSize);
                     });
                 }
-                wait_vmcnt<Q>();  // plane p + 1, sent before these Q stores, has landed
             } else {
-                wait_vmcnt<0>();
+                wait_vmcnt();
             }
             each<0, Q>([&](auto s) {
                 if constexpr (L::ez[s] == 0) hold0[s] = o[s];
                 if constexpr (L::ez[s] > 0) { up2[s] = up1[s]; up1[s] = o[s]; }
             });
         } else {
-            wait_vmcnt<0>();
+            wait_vmcnt();
         }
         tp = t;
     }
