@@ -21,7 +21,6 @@ namespace tlbm {
 constexpr int kUnit = 32;           // samples a wavefront takes at a time
 constexpr int kGradWaves = 4;       // wavefronts of a training workgroup
 constexpr int kGradBlocks = 256;    // at most one training workgroup per CU
-constexpr int kGradLen = kMlpParams + 1;  // + loss
 // offsets of the flat parameters
 constexpr int kB1 = kMlpH * kMlpIn, kW2 = kB1 + kMlpH, kB2 = kW2 + kMlpH * kMlpH, kW3 = kB2 + kMlpH,
               kB3 = kW3 + kMlpH;
@@ -33,8 +32,8 @@ __device__ inline uint64_t mix64(uint64_t x) {  // splitmix64 finaliser
     return x ^ (x >> 31);
 }
 
-// Partial gradient of one workgroup's samples.  mode 0: sample i of the batch
-// is index first + i; mode 1: a hashed index.
+// Partial gradient and loss of one workgroup's samples.  mode 0: sample i of the
+// batch is index first + i; mode 1: a hashed index.
 //
 // All five products are v_mfma_f32_32x32x2_f32 (lane l supplies A[l%32][g] and
 // B[g][l%32], g = l/32; lane l holds, in register 4q + r, row 8q + 4g + r of
@@ -46,14 +45,16 @@ __device__ inline uint64_t mix64(uint64_t x) {  // splitmix64 finaliser
 // a sample and read by columns, within the wavefront.  b1 is the weight of an
 // eighth input 1, so its gradient is that of W1.
 //
-// Bound by the MFMA rate: 68 products of 64 cycles per 32 samples, 3.6 us for
-// 65536 samples.  One thread per sample with the weights in LDS took 46 us
-// (an LDS read per multiply-add), and a fold by one thread per parameter
+// 65536 samples take 20 us.  The 68 products of 64 cycles per 32 samples are
+// 3.6 us of that; the rest is what a wavefront's two units do not hide: the
+// operands' loads, the samples' hashed indexes and gathers, the LDS passes and
+// the wavefronts' sums.  One thread per sample with the weights in LDS took
+// 46 us (an LDS read per multiply-add), and a fold by one thread per parameter
 // 159 us (512 dependent loads).
 __global__ void __launch_bounds__(kGradWaves * 64)
 k_mlp_grad(const float *__restrict__ X, const float *__restrict__ Tg, int64_t M, int64_t first,
            int mode, uint64_t seed, int64_t step, int64_t batch, const float *__restrict__ params,
-           float *__restrict__ partial) {
+           float *__restrict__ partial, double *__restrict__ losses) {
     constexpr int S = kMlpH + 4;  // row of a sample in LDS: 16-byte aligned, banks spread
     struct Wave {
         float d[kUnit * S];   // deltas by sample (d2, then d1)
@@ -61,7 +62,8 @@ k_mlp_grad(const float *__restrict__ X, const float *__restrict__ Tg, int64_t M,
         float x[kUnit * 12];  // inputs by sample
     };
     __shared__ alignas(16) Wave sw[kGradWaves];
-    __shared__ float sum[kGradLen];
+    __shared__ float sum[kMlpParams];
+    __shared__ double loss_sum;
     const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, c = l & 31, g = l >> 5;
     Wave &W = sw[wave];
     const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -83,7 +85,8 @@ k_mlp_grad(const float *__restrict__ X, const float *__restrict__ Tg, int64_t M,
     }
     const float b3 = params[kB3];
     f32x16 gW2 = zero, gW1 = zero, gb2 = zero, gw3 = zero;
-    float gb3 = 0.f, loss = 0.f;
+    float gb3 = 0.f;
+    double loss = 0.0;
     const int64_t units = (batch + kUnit - 1) / kUnit, stride = int64_t(gridDim.x) * kGradWaves;
     for (int64_t un = int64_t(blockIdx.x) * kGradWaves + wave; un < units; un += stride) {
         const int64_t pos = un * kUnit + c;
@@ -118,7 +121,7 @@ k_mlp_grad(const float *__restrict__ X, const float *__restrict__ Tg, int64_t M,
         const float r = live ? y - target : 0.f;
         const float dz = r / (1.f + expf(-z)) / float(batch);
         if (g == 0) {
-            loss += 0.5f * r * r;
+            loss += double(0.5f * r * r);
             gb3 += dz;
         }
         f32x16 d2;
@@ -168,12 +171,12 @@ k_mlp_grad(const float *__restrict__ X, const float *__restrict__ Tg, int64_t M,
         W.d[k * 64 + l] = gb2[k];
         W.h[k * 64 + l] = gw3[k];
     }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
+    for (int off = 16; off > 0; off >>= 1) {  // lanes 32-63 hold none
         gb3 += __shfl_xor(gb3, off, 64);
         loss += __shfl_xor(loss, off, 64);
     }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     float unit = 0.f;  // lanes 0-31: db2 of unit c; lanes 32-63: dw3
     {
         const float *src = (g == 0 ? W.d : W.h) + (4 * (c >> 3) + (c & 3)) * 64 + 32 * ((c >> 2) & 1);
@@ -192,38 +195,45 @@ k_mlp_grad(const float *__restrict__ X, const float *__restrict__ Tg, int64_t M,
             }
             add((g == 0 ? kB2 : kW3) + c, unit);
             if (l == 0) add(kB3, gb3);
-            if (l == 1) add(kMlpParams, loss);
+            if (l == 1) loss_sum = v == 0 ? loss : loss_sum + loss;
         }
         __syncthreads();
     }
-    float *out = partial + size_t(blockIdx.x) * kGradLen;
-    for (int k = threadIdx.x; k < kGradLen; k += kGradWaves * 64) out[k] = sum[k];
+    float *out = partial + size_t(blockIdx.x) * kMlpParams;
+    for (int k = threadIdx.x; k < kMlpParams; k += kGradWaves * 64) out[k] = sum[k];
+    if (threadIdx.x == 0) losses[blockIdx.x] = loss_sum;
 }
 
-// Fold the partial gradients in block order; with adam != 0 apply Adam.
-// grad_out (may be null) receives the folded gradient, loss_out the mean loss.
-// A workgroup folds 16 parameters: slice i of its 16 slices of 16 threads adds
-// every 16th partial, then the slices' sums are added in order.
+// Fold the partial gradients in double; with adam != 0 apply Adam.  grad_out
+// (may be null) receives the folded gradient, loss_out the mean loss.  A
+// workgroup folds 16 parameters, the last one the loss: slice i of its 16
+// slices of 16 threads adds partials i, i + 16, ..., then the slices' sums are
+// added in order.
+constexpr int kFoldBlocks = (kMlpParams + 15) / 16 + 1;
 __global__ void __launch_bounds__(256)
-k_mlp_fold_adam(const float *__restrict__ partial, int nblocks, int64_t batch, int adam,
-                float *__restrict__ params, float *__restrict__ mom, float *__restrict__ vel,
+k_mlp_fold_adam(const float *__restrict__ partial, const double *__restrict__ losses, int nblocks, int64_t batch,
+                int adam, float *__restrict__ params, float *__restrict__ mom, float *__restrict__ vel,
                 float lr, float c1, float c2, float *__restrict__ grad_out,
                 double *__restrict__ loss_out) {
     __shared__ double part[16][17];
     const int p = threadIdx.x & 15, slice = threadIdx.x >> 4;
     const int k = blockIdx.x * 16 + p;
-    double acc = 0.0;  // the loss is summed in double; a double sum of floats costs nothing here
-    if (k <= kMlpParams) {
+    const bool mean = blockIdx.x == kFoldBlocks - 1 && p == 0;
+    double acc = 0.0;
+    if (k < kMlpParams) {
 #pragma unroll 4
-        for (int b = slice; b < nblocks; b += 16) acc += double(partial[size_t(b) * kGradLen + k]);
+        for (int b = slice; b < nblocks; b += 16) acc += double(partial[size_t(b) * kMlpParams + k]);
+    } else if (mean) {
+#pragma unroll 4
+        for (int b = slice; b < nblocks; b += 16) acc += losses[b];
     }
     part[slice][p] = acc;
     __syncthreads();
-    if (slice != 0 || k > kMlpParams) return;
+    if (slice != 0 || (k >= kMlpParams && !mean)) return;
     double total = 0.0;
 #pragma unroll
     for (int i = 0; i < 16; ++i) total += part[i][p];
-    if (k == kMlpParams) {
+    if (mean) {
         *loss_out = total / double(batch);
         return;
     }
@@ -284,7 +294,7 @@ struct tlbm_mlp_trainer {
     int64_t n = 0;
     float *X = nullptr, *T = nullptr, *params = nullptr, *mom = nullptr, *vel = nullptr;
     float *partial = nullptr, *grad = nullptr;
-    double *loss = nullptr;
+    double *loss = nullptr, *losses = nullptr;  // of the batch; of the training workgroups
     int max_batch = 0, max_blocks = 0;
     int64_t steps = 0;
     uint64_t seed = 0;
@@ -317,7 +327,8 @@ int tlbm_mlp_trainer_create(const float *x, const float *t, int64_t n, const flo
         hipMalloc(&tr->vel, sizeof(float) * P) != hipSuccess ||
         hipMalloc(&tr->grad, sizeof(float) * P) != hipSuccess ||
         hipMalloc(&tr->loss, sizeof(double)) != hipSuccess ||
-        hipMalloc(&tr->partial, sizeof(float) * size_t(tr->max_blocks) * tlbm::kGradLen) != hipSuccess)
+        hipMalloc(&tr->partial, sizeof(float) * size_t(tr->max_blocks) * P) != hipSuccess ||
+        hipMalloc(&tr->losses, sizeof(double) * size_t(tr->max_blocks)) != hipSuccess)
         return bail(mfail(TLBM_ENOMEM, "device allocation failed"));
     if (hipMemcpy(tr->X, x, sizeof(float) * size_t(n) * tlbm::kMlpIn, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(tr->T, t, sizeof(float) * size_t(n), hipMemcpyHostToDevice) != hipSuccess ||
@@ -333,7 +344,8 @@ int tlbm_mlp_trainer_destroy(tlbm_mlp_trainer *tr) {
     if (!tr) return TLBM_OK;
     if (tr->stream) (void)hipStreamSynchronize(tr->stream);
     for (void *p : {(void *)tr->X, (void *)tr->T, (void *)tr->params, (void *)tr->mom,
-                    (void *)tr->vel, (void *)tr->partial, (void *)tr->grad, (void *)tr->loss})
+                    (void *)tr->vel, (void *)tr->partial, (void *)tr->grad, (void *)tr->loss,
+                    (void *)tr->losses})
         if (p) (void)hipFree(p);
     if (tr->stream) (void)hipStreamDestroy(tr->stream);
     delete tr;
@@ -350,12 +362,12 @@ int tlbm_mlp_trainer_step(tlbm_mlp_trainer *tr, int steps, int batch, float lr, 
         ++tr->steps;
         hipLaunchKernelGGL(tlbm::k_mlp_grad, dim3(nb), dim3(tlbm::kGradWaves * 64), 0, tr->stream, tr->X, tr->T,
                            tr->n, int64_t(0), 1, tr->seed, tr->steps, int64_t(batch), tr->params,
-                           tr->partial);
+                           tr->partial, tr->losses);
         MLP_HIP(hipGetLastError());
         const float c1 = 1.f - std::pow(0.9f, float(tr->steps));
         const float c2 = 1.f - std::pow(0.999f, float(tr->steps));
-        hipLaunchKernelGGL(tlbm::k_mlp_fold_adam, dim3((tlbm::kGradLen + 15) / 16), dim3(256),
-                           0, tr->stream, tr->partial, nb, int64_t(batch), 1, tr->params, tr->mom,
+        hipLaunchKernelGGL(tlbm::k_mlp_fold_adam, dim3(tlbm::kFoldBlocks), dim3(256),
+                           0, tr->stream, tr->partial, tr->losses, nb, int64_t(batch), 1, tr->params, tr->mom,
                            tr->vel, lr, c1, c2, (float *)nullptr, tr->loss);
         MLP_HIP(hipGetLastError());
     }
@@ -374,10 +386,10 @@ int tlbm_mlp_trainer_loss_grad(tlbm_mlp_trainer *tr, int64_t first, int64_t coun
         return mfail(TLBM_EINVAL, "count larger than the trainer's max_batch");
     const int nb = grad_blocks(count);
     hipLaunchKernelGGL(tlbm::k_mlp_grad, dim3(nb), dim3(tlbm::kGradWaves * 64), 0, tr->stream, tr->X, tr->T, tr->n,
-                       first, 0, tr->seed, int64_t(0), count, tr->params, tr->partial);
+                       first, 0, tr->seed, int64_t(0), count, tr->params, tr->partial, tr->losses);
     MLP_HIP(hipGetLastError());
-    hipLaunchKernelGGL(tlbm::k_mlp_fold_adam, dim3((tlbm::kGradLen + 15) / 16), dim3(256), 0,
-                       tr->stream, tr->partial, nb, count, 0, tr->params, tr->mom, tr->vel, 0.f, 1.f,
+    hipLaunchKernelGGL(tlbm::k_mlp_fold_adam, dim3(tlbm::kFoldBlocks), dim3(256), 0,
+                       tr->stream, tr->partial, tr->losses, nb, count, 0, tr->params, tr->mom, tr->vel, 0.f, 1.f,
                        1.f, tr->grad, tr->loss);
     MLP_HIP(hipGetLastError());
     MLP_HIP(hipMemcpyAsync(grad, tr->grad, sizeof(float) * tlbm::kMlpParams, hipMemcpyDeviceToHost, tr->stream));
