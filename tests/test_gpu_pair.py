@@ -1,11 +1,13 @@
 """The two-step pass (tlbm_amd/csrc/lbm_pair.h) against single steps.
 
 A call of several steps takes them two at a time where pair_plan says so, a
-call of one step never does, so step(7) and seven calls step(1) from one
-random state compare the two.  Lattices just large enough for the pass: last
-tiles that overhang the lattice in x and y, z segments of unequal length, the
-periodic wrap in x, y and z across tiles, walls, an obstacle across a tile's
-edge, inlet (with and without a profile) and outlet, and both tile widths.
+call of one step never does, so a call of n steps and n calls of one from one
+random state compare the two.  One lattice for every kernel that is built
+(velocity set, storage, tile, with and without the network; test_pair_plan.py
+holds which tile each takes and that none is left out), just large enough for
+the pass: last tiles that overhang the lattice in x and y, z segments of
+unequal length, the periodic wrap in x, y and z across tiles, walls, an
+obstacle across a tile's edge, inlet (with and without a profile) and outlet.
 
 Both run the same node update on the same values, with every rounding written
 out, so they agree bit for bit in every storage, with the network too."""
@@ -18,23 +20,34 @@ from tlbm_amd.workloads import DEFAULT_NETWORK
 
 pytestmark = pytest.mark.gpu
 
-CASES = [  # q, storage, dims, cs, network, inlet profile
-    (19, "f32", (100, 78, 67), 0.0, False, True),
-    (19, "f32", (28, 173, 117), 0.1, False, False),
-    (19, "f64", (94, 71, 90), 0.1, False, False),
-    (15, "f64", (64, 64, 97), 0.0, False, True),
-    (15, "f32", (124, 50, 90), 0.1, False, False),
-    (27, "f32", (60, 95, 101), 0.1, False, False),
-    (19, "f32x", (124, 65, 64), 0.0, False, False),
-    (27, "f32x", (124, 95, 90), 0.1, False, True),
-    (19, "f32", (124, 118, 132), 0.0, True, True),
-    (27, "f32", (128, 112, 107), 0.0, True, False),
+CASES = [  # q, storage, tile, dims, cs, network, inlet profile
+    (15, "f64", 0, (188, 59, 27), 0.0, False, True),
+    (15, "f32", 0, (188, 49, 67), 0.1, False, False),
+    (15, "f32", 1, (92, 103, 27), 0.0, False, True),
+    (15, "f32", 0, (252, 206, 91), 0.0, True, False),
+    (15, "f32", 1, (252, 111, 127), 0.0, True, True),
+    (15, "f32x", 0, (252, 47, 31), 0.0, False, False),
+    (15, "f32x", 1, (220, 47, 35), 0.0, False, True),
+    (19, "f64", 0, (92, 35, 111), 0.0, False, True),
+    (19, "f64", 0, (62, 191, 70), 0.1, False, False),
+    (19, "f32", 0, (124, 39, 61), 0.0, False, True),
+    (19, "f32", 1, (120, 41, 63), 0.0, False, False),
+    (19, "f32", 1, (248, 53, 47), 0.1, False, False),
+    (19, "f32", 0, (316, 38, 168), 0.0, True, True),
+    (19, "f32", 1, (220, 251, 35), 0.0, True, False),
+    (19, "f32x", 0, (380, 34, 47), 0.0, False, False),
+    (19, "f32x", 1, (220, 47, 53), 0.0, False, True),
+    (19, "f32x", 1, (252, 159, 79), 0.1, False, False),
+    (27, "f32", 0, (188, 54, 45), 0.0, False, False),
+    (27, "f32", 0, (124, 142, 41), 0.1, False, True),
+    (27, "f32", 1, (92, 123, 35), 0.0, False, True),
+    (27, "f32", 0, (316, 135, 134), 0.0, True, False),
+    (27, "f32", 1, (124, 143, 159), 0.0, True, True),
+    (27, "f32x", 0, (124, 47, 125), 0.0, False, True),
 ]
 
 
-@pytest.mark.parametrize("q,storage,dims,cs,network,profile", CASES,
-                         ids=[f"q{c[0]}-{c[1]}-{'x'.join(map(str, c[2]))}{'-net' if c[4] else ''}" for c in CASES])
-def test_two_step_pass_matches_single_steps(gpu_lib, q, storage, dims, cs, network, profile):
+def _compare(q, storage, dims, cs, network, profile, steps, **kw):
     nx, ny, nz = dims
     print(f"q={q} {storage} {dims} cs={cs} network={network}", flush=True)
     nd = geometry.channel(nx, ny, nz, walls=("left", "bottom") if q == 19 else (),
@@ -43,8 +56,8 @@ def test_two_step_pass_matches_single_steps(gpu_lib, q, storage, dims, cs, netwo
     rng = np.random.default_rng(q + nx)
     out = []
     f0 = None
-    for calls in ((7,), (1,) * 7):
-        with Lattice(q, nx, ny, nz, nd, omega=1.0 / 0.56, u_lbm=0.04, cs=cs, storage=storage) as lat:
+    for calls in ((steps,), (1,) * steps):
+        with Lattice(q, nx, ny, nz, nd, omega=1.0 / 0.56, u_lbm=0.04, cs=cs, storage=storage, **kw) as lat:
             if network:
                 lat.set_closure(*closure.split_closure(closure.load_network(DEFAULT_NETWORK))[0])
             if profile:
@@ -61,3 +74,18 @@ def test_two_step_pass_matches_single_steps(gpu_lib, q, storage, dims, cs, netwo
     assert np.array_equal(fa, fb)
     assert all(np.array_equal(ma[k], mb[k]) for k in ma)
     assert ra == rb and sa == sb
+
+
+@pytest.mark.parametrize("q,storage,tile,dims,cs,network,profile", CASES,
+                         ids=[f"q{c[0]}-{c[1]}-tile{c[2]}-{'x'.join(map(str, c[3]))}{'-net' if c[5] else ''}"
+                              for c in CASES])
+def test_two_step_pass_matches_single_steps(gpu_lib, q, storage, tile, dims, cs, network, profile):
+    _compare(q, storage, dims, cs, network, profile, 7)
+
+
+@pytest.mark.parametrize("storage", ["f64", "f32", "f32x"])
+@pytest.mark.parametrize("steps,kw", [(2, {}), (4, {}), (8, {}), (5, {"dynamics": 2}), (6, {"exact_weights": True})],
+                         ids=["2", "4", "8", "no-relaxation", "exact-weights"])
+def test_counts_and_options(gpu_lib, storage, steps, kw):
+    dims = {"f64": (92, 35, 111), "f32": (120, 41, 63), "f32x": (220, 47, 53)}[storage]  # of CASES
+    _compare(19, storage, dims, 0.0, False, True, steps, **kw)

@@ -2,8 +2,6 @@
 // kernels_f64.hip and kernels_f32.hip.
 #pragma once
 
-#include <type_traits>
-
 #include "launch.h"
 #include "lbm_aux.h"
 
@@ -94,19 +92,17 @@ struct Launch {
 
     // f(tile k of the pair pass); false if there is none
     template <class L, class F>
-    static bool pair_tile(int k, F f) {
-        using T0 = typename PairShapes<L, ST>::T0;
-        using T1 = typename PairShapes<L, ST>::T1;
-        if constexpr (!std::is_void_v<T0>)
-            if (k == 0) { f(T0{}); return true; }
-        if constexpr (!std::is_void_v<T1>)
-            if (k == 1) { f(T1{}); return true; }
+    static bool pair_tile_of(int k, F f) {
+        if constexpr (pair_tile(L::Q, ST, 0).tx != 0)
+            if (k == 0) { f(PairTile<L, ST, 0>{}); return true; }
+        if constexpr (pair_tile(L::Q, ST, 1).tx != 0)
+            if (k == 1) { f(PairTile<L, ST, 1>{}); return true; }
         return false;
     }
     template <class L>
     static hipError_t lbm_pair_l(const void *fin, void *fout, const uint8_t *nd, const PairPlan &pl,
                                  const StepArgs &a, hipStream_t s) {
-        const bool found = pair_tile<L>(pl.shape, [&](auto tile) {
+        const bool found = pair_tile_of<L>(pl.shape, [&](auto tile) {
             using TL = decltype(tile);
             const dim3 grid(pl.ntx * pl.nty * pl.nseg), block(TL::BS);
             const st *in = static_cast<const st *>(fin);
@@ -125,21 +121,6 @@ struct Launch {
                                const PairPlan &pl, const StepArgs &a, hipStream_t s) {
         TLBM_BY_LATTICE(lbm_pair_l, fin, fout, nd, pl, a, s)
     }
-    template <class L>
-    static bool pair_shape_l(int k, PairShape &out) {
-        return pair_tile<L>(k, [&](auto tile) {
-            using TL = decltype(tile);
-            out = {TL::TX, TL::TY, TL::V};
-        });
-    }
-    static bool pair_shape(int lattice, int k, PairShape &out) {
-        switch (lattice) {
-        case 15: return pair_shape_l<D3Q15>(k, out);
-        case 19: return pair_shape_l<D3Q19>(k, out);
-        default: return pair_shape_l<D3Q27>(k, out);
-        }
-    }
-
     template <class L>
     static hipError_t init_rest_l(void *fout, const StepArgs &a, hipStream_t s) {
         hipLaunchKernelGGL((k_init_rest<L, ST>), dim3(blocks_for(a.N)), dim3(kBlock), 0, s,
@@ -219,7 +200,7 @@ struct Launch {
     }
 
     static const LaunchOps &table() {
-        static const LaunchOps t = {&lbm, &lbm_pair, &pair_shape, &init_rest, &init_macros, &get_populations,
+        static const LaunchOps t = {&lbm, &lbm_pair, &init_rest, &init_macros, &get_populations,
                                     &set_populations, &forces, &reduce, &box_filter, int(sizeof(T))};
         return t;
     }

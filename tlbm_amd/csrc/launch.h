@@ -20,7 +20,6 @@ struct LaunchOps {
     // two steps in one pass (lbm_pair.h)
     hipError_t (*lbm_pair)(int lattice, const void *fin, void *fout, const uint8_t *nd,
                            const PairPlan &plan, const StepArgs &a, hipStream_t s);
-    bool (*pair_shape)(int lattice, int k, PairShape &out);  // its k-th tile; false: there is none
     hipError_t (*init_rest)(int lattice, void *fout, const StepArgs &a, hipStream_t s);
     hipError_t (*init_macros)(int lattice, void *fout, const double *mac, const StepArgs &a,
                               hipStream_t s);

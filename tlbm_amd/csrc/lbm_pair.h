@@ -41,39 +41,23 @@ constexpr int pair_slot(int s) {
     return n;
 }
 
-// A kernel's tile: TX x TY own columns, the threads and the LDS they take.
-template <class L, int ST, int TX_, int TY_>
+// The K-th tile's kernel: TX x TY own columns, the threads and the LDS they take.
+template <class L, int ST, int K>
 struct PairTile {
-    static constexpr int TX = TX_, TY = TY_;
+    static constexpr PairShape kShape = pair_tile(L::Q, ST, K);
+    static constexpr int TX = kShape.tx, TY = kShape.ty;
     static constexpr int W = TX + 2, H = TY + 2;      // with the rim
     static constexpr int kOwn = (TX * TY + 63) / 64 * 64;  // the own columns' threads, whole wavefronts
     static constexpr int kRim = 2 * W + 2 * TY;
     static constexpr int BS = (kOwn + kRim + 63) / 64 * 64;
     static constexpr int kSize = int(sizeof(typename StorageT<ST>::st));
-    static constexpr int V = 16 / kSize;              // values of a 16-byte load
+    static constexpr int V = kShape.v;                // values of a 16-byte load
+    static_assert(V * kSize == 16, "whole 16-byte loads");
     static constexpr int SW = TX + 2 * V;             // staged row: x0 - V .. x0 + TX + V - 1
     static constexpr int kStage = L::Q * H * SW;      // staged values
     static constexpr int NS = pair_slot<L>(L::Q);
     static constexpr size_t kLds = size_t(kStage + NS * W * H) * kSize;
     static_assert(kLds <= 160 * 1024, "LDS of a CU");
-};
-
-// The tiles a storage and lattice are built for: T0, and T1 for lattices whose
-// width T0 fits badly.  Each is as large as LDS (160 KiB) and the registers
-// of one workgroup per CU allow.  FP16 and D3Q27 FP64 have none: FP16's pair
-// of steps is bound by VALU issue and takes as long as two steps (D3Q19
-// 128x128x512: 103 against 2 x 102 us per 2 x 2 steps), D3Q27 FP64 needs more
-// than 256 registers.
-template <class L, int ST> struct PairShapes { using T0 = void; using T1 = void; };
-template <> struct PairShapes<D3Q15, ST_F64> { using T0 = PairTile<D3Q15, ST_F64, 32, 12>; using T1 = void; };
-template <> struct PairShapes<D3Q19, ST_F64> { using T0 = PairTile<D3Q19, ST_F64, 32, 12>; using T1 = void; };
-template <class L> struct PairShapes<L, ST_F32> {
-    using T0 = PairTile<L, ST_F32, 64, L::Q == 27 ? 8 : 13>;
-    using T1 = PairTile<L, ST_F32, 32, L::Q == 27 ? 18 : 28>;
-};
-template <class L> struct PairShapes<L, ST_F32X> {
-    using T0 = PairTile<L, ST_F32X, 64, L::Q == 27 ? 4 : 8>;
-    using T1 = PairTile<L, ST_F32X, 32, L::Q == 27 ? 12 : 20>;
 };
 
 // s_waitcnt vmcnt(0), other counters free: every load and store sent has landed.
@@ -102,6 +86,7 @@ k_lbm_pair(const typename StorageT<ST>::st *__restrict__ fin, typename StorageT<
     using S = StorageT<ST>;
     using T = typename S::T;
     using st = typename S::st;
+    static_assert(ST != ST_F16, "no stochastic rounding here");
     constexpr int Q = L::Q;
     constexpr uint32_t kSize = sizeof(st);
     constexpr int CB = S::kCB;
@@ -227,8 +212,7 @@ k_lbm_pair(const typename StorageT<ST>::st *__restrict__ fin, typename StorageT<
         each<0, Q>([&](auto s) { f[s] = S::in(o[s], s, a); });
         uint32_t g = wrapz(p) * a.nxny + gxy;
         update(f, t, g);
-        uint32_t rs = ST == ST_F16 ? round_stream(g, a.step) : 0u;
-        each<0, Q>([&](auto s) { o[s] = S::step_out(f[s], s, a, rs + uint32_t(s) * kStreamStep); });
+        each<0, Q>([&](auto s) { o[s] = S::step_out(f[s], s, a, 0u); });
         if (live) {
             each<0, Q>([&](auto s) {
                 if constexpr (pair_moves<L>(s)) wp[pair_slot<L>(s) * (W * H)] = o[s];
@@ -247,7 +231,6 @@ k_lbm_pair(const typename StorageT<ST>::st *__restrict__ fin, typename StorageT<
                 });
                 g = uint32_t(p - 1) * a.nxny + gxy;
                 update(f, tp, g);
-                rs = ST == ST_F16 ? round_stream(g, a.step + 1) : 0u;
                 // the plane's first chunk by a descriptor, the rest by the lane
                 const uint32_t first = uint32_t(p - 1) * a.nxny, c = first >> CB;
                 const uint64_t back = uint64_t(c) * (Q * CH * kSize);
@@ -257,8 +240,8 @@ k_lbm_pair(const typename StorageT<ST>::st *__restrict__ fin, typename StorageT<
                 wait_vmcnt();  // plane p + 1 has landed (ahead of the stores, which then need no count)
                 if (own) {
                     each<0, Q>([&](auto s) {
-                        RawBuf<st>::template store<kAuxNT>(S::step_out(f[s], s, a, rs + uint32_t(s) * kStreamStep),
-                                                           rsrc, off, uint32_t(s) * CH * kSize);
+                        RawBuf<st>::template store<kAuxNT>(S::step_out(f[s], s, a, 0u), rsrc, off,
+                                                           uint32_t(s) * CH * kSize);
                     });
                 }
             } else {

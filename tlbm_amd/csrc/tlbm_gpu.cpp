@@ -323,10 +323,9 @@ int tlbm_gpu_create(const tlbm_params *p, const uint8_t *nd_type, tlbm_gpu **out
             cus = 0;
         for (int net = 0; net < 2; ++net)
             h->pair[net] = !has_lid && cus > 0 && (net == 0 || p->storage == TLBM_STORAGE_F32) &&
-                           tlbm::pair_plan(
-                               a.nx, a.ny, a.nz, Q, int(storage_bytes(p->storage)), net != 0, uint32_t(cus),
-                               [&](int k, tlbm::PairShape &s) { return h->ops->pair_shape(Q, k, s); },
-                               &h->plan[net]);
+                           tlbm::pair_plan(a.nx, a.ny, a.nz, Q, p->storage,
+                                           net ? tlbm::kRateNetwork : a.smag ? tlbm::kRateSmagorinsky : tlbm::kRateBgk,
+                                           uint32_t(cus), &h->plan[net]);
     }
     hipError_t e;
     if ((e = hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking)) != hipSuccess)
