@@ -9,7 +9,8 @@ tau = 0.55, starting from rest (f = w).
 
 A step is one fused stream-collide update of the whole lattice with the
 populations resident in HBM; FP32, FP64 and FP32X take two steps per launch
-(all but a call's last one or two), FP16 one.  The headline `value` is MLUPS with FP32
+(all but a call's last one or two), FP16 one; the library counts the launches.
+The headline `value` is MLUPS with FP32
 storage (nx*ny*nz*steps / wall time of the timed steps); FP64, FP16 (f - w)
 and FP32X storage run the same timed steps, reported under `variants`.
 After the timed region every storage runs the configuration's full 20000
@@ -19,8 +20,8 @@ on-device sums) and the reference's own validation metric, the relative
 1-norm difference of the speed |u| over all nodes (python/validate.py:33-43),
 against the FP64 run.  `roofline` prices the FP32 kernel at the 2*Q*4 = 152
 bytes that each node's populations take to read and write once per launch,
-i.e. 76 per lattice update, against 8 TB/s, with the average duration of a
-step from HIP events on the stream the kernel runs on.
+i.e. 152 * launches / steps per lattice update, against 8 TB/s, with the
+average duration of a step from HIP events on the stream the kernel runs on.
 `cpu_baseline` times the reference's own MPI executable (built from its
 sources into oracle/_ref) on the host's physical cores (those this process
 may run on, at most its CPU share) for 200 steps of the same lattice, or the
@@ -47,8 +48,6 @@ from tlbm_amd.gpu import BYTES_PER_VALUE, Lattice  # noqa: E402
 
 METRIC = "D3Q19 MLUPS & %HBM roofline, FP32/FP16 vs FP64 at stated L2 error"
 PEAK_HBM_GBS = 8000.0
-# steps of the timed lattice that one launch takes
-STEPS_PER_LAUNCH = {"f64": 2, "f32": 2, "f32x": 2, "f16": 1}
 Q = 19
 NX, NY, NZ = 128, 128, 512
 TAU = 0.55
@@ -66,13 +65,16 @@ def run_gpu(storage, nd, steps, warmup):
     with Lattice(Q, NX, NY, NZ, nd, storage=storage, **kw) as lat:
         lat.step(warmup)
         lat.sync()
+        before = lat.passes()
         t0 = time.perf_counter()
         ms_events = lat.step_timed(steps)
         wall = time.perf_counter() - t0
+        passes = lat.passes() - before
     n = NX * NY * NZ
     return {
         "wall_s": wall,
         "kernel_ms": ms_events / steps,
+        "launches": passes,
         "mlups": n * steps / wall / 1e6,
     }
 
@@ -279,8 +281,9 @@ def main():
     head = storages[0]
     h = res[head]
     n = NX * NY * NZ
+
     def bytes_per_update(st):
-        return 2 * Q * BYTES_PER_VALUE[st] // STEPS_PER_LAUNCH[st]
+        return round(2 * Q * BYTES_PER_VALUE[st] * res[st]["launches"] / args.steps, 3)
 
     b_alg = bytes_per_update(head)
     achieved = b_alg * n / (h["kernel_ms"] * 1e-3) / 1e9
@@ -288,7 +291,7 @@ def main():
     for st, r in res.items():
         variants[st] = {"mlups": round(r["mlups"], 1), "kernel_ms": round(r["kernel_ms"], 5),
                         "bytes_per_update": bytes_per_update(st),
-                        "steps_per_launch": STEPS_PER_LAUNCH[st],
+                        "launches": r["launches"],
                         "hbm_frac": round(bytes_per_update(st) * n / (r["kernel_ms"] * 1e-3)
                                           / 1e9 / PEAK_HBM_GBS, 4)}
     if args.accuracy_steps > 0:

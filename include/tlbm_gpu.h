@@ -83,6 +83,11 @@ int tlbm_gpu_step_timed(tlbm_gpu *h, int nsteps, double *ms);
 /* Wait for queued work. */
 int tlbm_gpu_sync(tlbm_gpu *h);
 
+/* Passes over the lattice that its steps have taken since it was created: a
+ * call of several steps may take two of them in one read and write of the
+ * populations.  No reference counterpart: for pricing a measured time. */
+int tlbm_gpu_step_passes(const tlbm_gpu *h, uint64_t *passes);
+
 /* ux, uy, uz, rho of the last step, as TLBM_Partition::write_data dumps
  * them (src/TLBM_Partition.cpp:608-650): moments after the boundary rule
  * (solid u = 0, inlet u = (0,0,u_lbm), outlet rho = rho_lbm).  Each array

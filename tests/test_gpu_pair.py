@@ -89,3 +89,19 @@ def test_two_step_pass_matches_single_steps(gpu_lib, q, storage, tile, dims, cs,
 def test_counts_and_options(gpu_lib, storage, steps, kw):
     dims = {"f64": (92, 35, 111), "f32": (120, 41, 63), "f32x": (220, 47, 53)}[storage]  # of CASES
     _compare(19, storage, dims, 0.0, False, True, steps, **kw)
+
+
+@pytest.mark.parametrize("storage,nx,passes", [("f64", 92, {1: 1, 2: 2, 3: 2, 7: 4, 8: 5}), ("f16", 92, {1: 1, 7: 7}),
+                                               ("f64", 93, {7: 7})])
+def test_passes_are_counted(gpu_lib, storage, nx, passes):
+    """Two steps a pass but for a call's last one or two; one where rows are
+    no multiple of 16 bytes, in FP16 and while averages are on."""
+    with Lattice(19, nx, 35, 111, np.zeros(nx * 35 * 111, np.uint8), omega=1.2, storage=storage) as lat:
+        for steps, n in passes.items():
+            before = lat.passes()
+            lat.step(steps)
+            assert lat.passes() - before == n
+        lat.time_average(True)
+        before = lat.passes()
+        lat.step(7)
+        assert lat.passes() - before == 7

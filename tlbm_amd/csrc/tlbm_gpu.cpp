@@ -160,6 +160,7 @@ struct tlbm_gpu {
     bool copies = false;  // holds a share of the host copy rings
     long long steps_since_set = 0;
     uint64_t step_count = 0;  // steps since creation (FP16 rounding stream)
+    uint64_t passes = 0;      // passes over the lattice that they took
     hipStream_t stream = nullptr;
     double *fixed_partial = nullptr;  // this device's copy of `scratch`
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -419,6 +420,7 @@ static int queue_steps(tlbm_gpu *h, int nsteps) {
             if (e != hipSuccess) return fail(TLBM_EHIP, std::string("two steps: ") + hipGetErrorString(e));
             h->cur = 1 - h->cur;
             h->step_count += 2;
+            ++h->passes;
             h->steps_since_set += 2;
         }
     }
@@ -437,6 +439,7 @@ static int queue_steps(tlbm_gpu *h, int nsteps) {
                                    h->chunk_type, fused ? h->avg : nullptr, h->uy_head, h->args, h->stream);
         if (e != hipSuccess) return fail(TLBM_EHIP, std::string("stream-collide: ") + hipGetErrorString(e));
         h->cur = 1 - h->cur;
+        ++h->passes;
         ++h->steps_since_set;
         if (fused) ++h->avg_steps;
         if (h->avg_on && !fused) {
@@ -472,6 +475,12 @@ int tlbm_gpu_step_timed(tlbm_gpu *h, int nsteps, double *ms) {
 int tlbm_gpu_sync(tlbm_gpu *h) {
     if (int rc = check(h)) return rc;
     TLBM_HIP(hipStreamSynchronize(h->stream));
+    return TLBM_OK;
+}
+
+int tlbm_gpu_step_passes(const tlbm_gpu *h, uint64_t *passes) {
+    if (!h || !passes) return fail(TLBM_EINVAL, "null argument");
+    *passes = h->passes;
     return TLBM_OK;
 }
 

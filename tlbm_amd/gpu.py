@@ -229,6 +229,12 @@ class Lattice:
         _check(load_library().tlbm_gpu_box_filter(self._h, out.ctypes.data))
         return dict(zip(FILTER_PLANES, out.reshape(len(FILTER_PLANES), -1)))
 
+    def passes(self) -> int:
+        """Passes over the lattice that its steps have taken (some take two steps)."""
+        n = ctypes.c_uint64()
+        _check(load_library().tlbm_gpu_step_passes(self._h, ctypes.byref(n)))
+        return int(n.value)
+
     def memory_bytes(self) -> int:
         b = ctypes.c_uint64()
         _check(load_library().tlbm_gpu_memory_bytes(self._h, ctypes.byref(b)))

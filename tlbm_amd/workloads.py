@@ -118,11 +118,12 @@ def timed_run(lat: Lattice, steps: int, chunk: int, tag: str) -> float:
     return ms
 
 
-def _rate(N, Q, storage, steps, ms):
+def _rate(N, Q, storage, steps, ms, passes):
+    """passes: over the lattice that the steps took (some take two steps)."""
     mlups = N * steps / (ms * 1e3)
-    return {"mlups": mlups, "ms_per_step": ms / steps,
-            "hbm_gbs": mlups * 1e6 * 2 * Q * STORAGE_BYTES[storage] / 1e9,
-            "bytes_per_update": 2 * Q * STORAGE_BYTES[storage]}
+    per_update = 2 * Q * STORAGE_BYTES[storage] * passes / steps
+    return {"mlups": mlups, "ms_per_step": ms / steps, "hbm_gbs": mlups * 1e6 * per_update / 1e9,
+            "bytes_per_update": per_update}
 
 
 def _l2(a: dict, b: dict, mask) -> float:
@@ -191,7 +192,7 @@ def run_porous(n: int = 384, steps: int = 5000, chunk: int = 500, seed: int = 20
                      f"f32 {ms['f32'] / done:.3f}")
                 del m64, m32
         for st, lat in lats.items():
-            r = _rate(N, Q, st, steps, ms[st])
+            r = _rate(N, Q, st, steps, ms[st], lat.passes())
             r["mass"] = float(lat.reduce()["mass"])
             out["runs"][st] = r
     finally:
@@ -263,7 +264,7 @@ def run_cylinders(steps: int = 20000, chunk: int = 500,
                 _log(f"cylinders step {done}: {cp}")
                 del m
         for st, lat in lats.items():
-            out["runs"][st] = _rate(N, Q, "f64" if st == "f64p" else st, steps, ms[st])
+            out["runs"][st] = _rate(N, Q, "f64" if st == "f64p" else st, steps, ms[st], lat.passes())
     finally:
         for lat in lats.values():
             lat.close()
@@ -301,7 +302,8 @@ def _spheroid_run(dims, nd, body, storage, tau, steps, chunk, closure=None, cs=0
         _log(f"{tag}: {steps}/{steps} steps, {ms / steps:.3f} ms/step")
         m = lat.macros()
         red = lat.reduce()
-    r = _rate(nd.size, 19, storage, steps, ms)
+        passes = lat.passes()
+    r = _rate(nd.size, 19, storage, steps, ms, passes)
     r.update({"drag": drags[-1], "drag_mean": float(np.mean(drags)),
               "drag_samples": drags, "mass": red["mass"]})
     _log(f"{tag}: {r}")
@@ -391,8 +393,10 @@ def run_slab(gpus: int = 8, steps: int = 1000, chunk: int = 500, scale: int = 1,
             lat.init_from_macros(zero, zero, uz, np.ones(nd.size))
             lat.step(20)
             tag = f"slab {nx}x{ny}x{nzs} {storage}{'+network' if cl is not None else ''}"
+            before = lat.passes()
             ms = timed_run(lat, steps, chunk, tag)
-        r = _rate(nd.size, 19, storage, steps, ms)
+            passes = lat.passes() - before
+        r = _rate(nd.size, 19, storage, steps, ms, passes)
         face = 5 * nx * ny * STORAGE_BYTES[storage]
         r["face_bytes"] = face
         # modelled, not measured: the face's bytes over one link's bandwidth
