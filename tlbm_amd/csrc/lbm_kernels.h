@@ -922,7 +922,8 @@ __device__ inline T smagorinsky_omega(const T (&pi)[6], const StepArgs &a) {
 // float roundings: the D3Q27 weights sum to 1 in double but to 1 + 7.5e-9
 // in float, a mass source FP64 does not have.  The residue of mass m0 and
 // momentum m is taken out of f - feq as w_s (m0 + 3 e_s.m), which carries
-// that mass and momentum.  Where fluid is false n stays.
+// that mass and momentum.  Where fluid is false n stays.  STEP: see
+// equilibrium_dev (it sets u^2 alone: e.m is rounded alike in either).
 template <class L, bool STEP>
 __device__ inline void conserve(float (&n)[L::Q], const float (&w)[L::Q], bool fluid, float rho, float ux, float uy,
                                 float uz, const StepArgs &a) {
@@ -949,7 +950,7 @@ __device__ inline void conserve(float (&n)[L::Q], const float (&w)[L::Q], bool f
         if constexpr (x * x + y * y + z * z == 1)
             c = fma_t(3.0f * float(x + y + z), x ? mx : y ? my : mz, m0);
         else if constexpr (s != 0)
-            c = m0 + edot_scaled<L, s, STEP>(3.0f, mx, my, mz, Mx, My, Mz);
+            c = m0 + edot_scaled<L, s, true>(3.0f, mx, my, mz, Mx, My, Mz);
         n[s] = fma_t(-w[s], c, n[s]);
     });
 }
