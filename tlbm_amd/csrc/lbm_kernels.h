@@ -64,7 +64,8 @@ template <int ST> constexpr bool kClosureNTLoad = (ST == ST_F16);
 // the network's MFMA chain.  Measured on 128x128x512 (us per step, 4 waves ->
 // this): FP16 D3Q19 156.5 -> 149.1 (6), D3Q15 141.9 -> 130.8 (6), D3Q27
 // 316.8 -> 197.6 (5); FP32 D3Q19 216.5 -> 214.5 (5), D3Q15 181.9 -> 167.8
-// (6).  FP32 D3Q27 stays at 4: at 5 it spills (325 against 299 us).
+// (6).  FP32 D3Q27 stays at 4: at 5 (96 VGPRs) 128^3 takes 77.2 against 77.3 us,
+// 61x60x59 13.26 against 13.06.
 template <int ST, int Q>
 constexpr int kClosureWaves = Q == 27 ? (ST == ST_F16 ? 5 : 4) : (ST == ST_F32 && Q == 19 ? 5 : 6);
 // Most waves per SIMD the step is register-allocated for: FP32 D3Q19,

@@ -21,7 +21,16 @@
 // wavefronts while it is still on its way, which holds up the L1.
 //
 // Each node runs the very update of k_lbm (NET: of k_lbm_closure) in both
-// steps, so the results are those of two single steps (FP64: bitwise).
+// steps in the same roundings, so the results are those of two
+// single steps bit for bit.
+//
+// us per step, single steps -> this: D3Q19 128x128x512 FP32 201.5 -> 148.8
+// (Smagorinsky 157.4, network 184.8), FP64 401 -> 317.5, FP32X 201 -> 159.8;
+// D3Q15 FP32 163.2 -> 122.3; D3Q27 FP32 192^3 248 -> 220.  What bounds it is
+// the one workgroup per CU, in lock step between three barriers a plane; LDS
+// and registers leave no room for a second to fill its waits.  No unit is
+// full: VALU issue is 47 (FP64) to 75 % busy (D3Q27 with Smagorinsky; 84 with
+// the network), LDS 8 to 11 % (26), and HBM moves 4.0 to 4.4 TB/s.
 #pragma once
 
 #include <type_traits>

@@ -17,9 +17,9 @@ struct PairShape {
 // The k-th tile (k = 0, 1) of a lattice of q directions in a storage
 // (TLBM_STORAGE_*); the second is for lattices whose width the first fits
 // badly.  Each is as large as LDS (160 KiB) and the registers of one workgroup
-// per CU allow.  FP16 and D3Q27 FP64 have none: FP16's pair of steps is bound
-// by VALU issue and takes as long as two steps (D3Q19 128x128x512: 103 against
-// 2 x 102 us per 2 x 2 steps), D3Q27 FP64 did not fit 256 registers.
+// per CU allow.  FP16 and D3Q27 FP64 have none: FP16's pair of steps takes
+// as long as two steps (D3Q19 128x128x512: 103 against 102 us per step), D3Q27
+// FP64 did not fit 256 registers when it was tried (806 against 502 us).
 constexpr PairShape pair_tile(int q, int storage, int k) {
     if (k < 0 || k > 1) return {};
     if (storage == 0 && q != 27 && k == 0) return {32, 12, 2};
